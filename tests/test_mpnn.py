@@ -263,6 +263,33 @@ def test_gpu_gradients_match_oracle(gpu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("side,copies", [(3, 2), (5, 64), (33, 64), (40, 128)])
+def test_gpu_gradients_of_repeated_graph(gpu, side, copies):
+  """A batch of 2^k copies of one graph has its loss and gradients: the mean
+  over rows does not change, every per-row term is scaled by a power of two
+  (so BF16 rounds it the same way), and only the FP32 sums over up to 409,600
+  rows run over more partials. Their rounding is at most about
+  sqrt(rows) * 2^-24 of the summed magnitudes, which the gradient's norm is a
+  few per cent of: 1e-4 covers it."""
+  from pgmax_amd import engine
+  from pgmax_amd import warmstart
+  torch = pytest.importorskip("torch")
+  w, lp, ev = _spin_glass(side, 17)
+  g = engine.Graph(w.to_engine_wiring())
+  net = warmstart.WarmStart(g, seed=3)
+  rng = np.random.default_rng(18)
+  t = np.stack([np.zeros(w.num_edge_states // 2), rng.normal(size=w.num_edge_states // 2)], 1)
+  args = [torch.as_tensor(np.asarray(a, np.float32).reshape(1, -1), device="cuda")
+          for a in (lp, ev, t)]
+  loss1, g1 = net.loss_and_grad(*args)
+  loss2, g2 = net.loss_and_grad(*[a.repeat(copies, 1) for a in args])
+  assert float((loss2 - loss1).abs()) <= 1e-5 * float(loss1)
+  assert float((g2 - g1).norm()) <= 1e-4 * float(g1.norm())
+  net.close()
+  g.close()
+
+
+@pytest.mark.gpu
 def test_gpu_gradients_deterministic(gpu):
   import torch
   from pgmax_amd import engine, warmstart
