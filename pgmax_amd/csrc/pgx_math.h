@@ -79,6 +79,24 @@ __device__ __forceinline__ float pgx_log_pos(float x) {
   return (ef * kLn2Lo + logm) + ef * kLn2Hi;
 }
 
+// pgx_log_pos for 1 <= x <= 2 (a log-sum-exp of two terms), the same bits:
+// frexp and the fold at sqrt(1/2) leave m = x, e = 0 below 2 sqrt(1/2) and
+// m = x / 2, e = 1 from there on, and with e = 0 the two terms e ln2 add
+// zeros. tests/test_oracle.py compares the two for every such x.
+__device__ __forceinline__ float pgx_log_1to2(float x) {
+  const bool upper = x >= 2.f * kSqrtHalf;
+  const float f = (upper ? x * 0.5f : x) - 1.f;
+  const float s = div_2pf(f);
+  const float z = s * s;
+  float q = 2.f / 11.f;
+  q = q * z + 2.f / 9.f;
+  q = q * z + 2.f / 7.f;
+  q = q * z + 2.f / 5.f;
+  q = q * z + 2.f / 3.f;
+  const float logm = f - s * (f - q * z);
+  return ((upper ? kLn2Lo : 0.f) + logm) + (upper ? kLn2Hi : 0.f);
+}
+
 // e^xc for an in-range xc (kExpLo <= xc <= kExpHi).
 __device__ __forceinline__ float pgx_exp_core(float xc) {
   const float k = rintf(xc * kInvLn2);

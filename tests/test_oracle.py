@@ -174,6 +174,24 @@ def test_f32_transcendentals_within_2p5_ulp():
   assert f32math.expm1(np.float32(-np.inf)) == -1
 
 
+def test_log_of_one_to_two_equals_log():
+  """The logarithm the kernels take of a two-term log-sum-exp (1 <= x <= 2,
+  no frexp: pgx_log_1to2) has the bits of the general one for every such x."""
+  F = np.float32
+  x = np.arange(np.float32(1).view(np.uint32), np.float32(2).view(np.uint32) + 1,
+                dtype=np.uint32).view(F)
+  upper = x >= F(2) * f32math.SQRT_HALF
+  f = np.where(upper, x * F(0.5), x) - F(1)
+  s = f / (F(2) + f)
+  z = s * s
+  q = np.full_like(z, f32math.D[11])
+  for k in (9, 7, 5, 3):
+    q = q * z + f32math.D[k]
+  logm = f - s * (f - q * z)
+  got = (np.where(upper, f32math.LN2_LO, F(0)) + logm) + np.where(upper, f32math.LN2_HI, F(0))
+  np.testing.assert_array_equal(got.view(np.uint32), f32math.log(x).view(np.uint32))
+
+
 def test_var_sum_order():
   """Degree <= 32: plain sequential scatter-add; higher degree: chunked, within rounding of the exact sum."""
   rng = np.random.default_rng(3)
