@@ -46,6 +46,8 @@ struct DevGraph {
   const int4* col_desc;        // per column chunk (null: chunk_desc, all chunks)
   const int4* row_desc;        // per row chunk
   const int4* heavy_desc;      // per heavy variable -- see Plan::heavy_desc
+  const int4* wide_desc;       // per variable of many states -- see Plan::wide_desc
+  int32_t num_wide;
   const int32_t* vh_group_h;
   const int32_t* vh_group_j;
   int32_t num_vh_groups;
@@ -1015,6 +1017,96 @@ static_assert(pair_lanes_lds(2) <= kPairLanesLds && pair_lanes_lds(3) <= kPairLa
                   pair_lanes_lds(7) <= kPairLanesLds,
               "S = 8 needs the most LDS");
 
+// Full pairwise tables of more than 8 states (s0 x s1, config p * s1 + q) on
+// one lane per edge state, for the per-phase factor kernel: lane k < s0 owns
+// row k, lane s0 + q column q, so the row and the column log-sum-exps of a
+// factor run at the same time in one set of lanes; 64 / (s0 + s1) factors
+// share a wavefront. The lanes read the table once, in order, form the
+// summaries (0 + x_a[p]) + x_b[q] + lp into the wavefront's LDS (sm, rows
+// padded to an odd pitch) and reduce row or column from there, over the same
+// operands in the same order as enum_general_wave; the damped messages and
+// per-edge maxima go through xs. Bound by latency: the general kernel walked
+// per-state config lists in global memory and finished each edge in one lane
+// (29.8 us an iteration on 5,384 factors 16 x 16); this form takes 9.8 us.
+// on: the lane has a factor; every lane of the wavefront must call it.
+template <bool kT0>
+__device__ __forceinline__ void pair_wide(const DevGraph& g, const Block& b, int32_t i, bool on,
+                                          int32_t k, const EngineIO& io, float t, float& dl,
+                                          float* xs, float* sm) {
+  constexpr int kAhead = 8;  // table loads in flight per lane
+  const int32_t s0 = b.s0, s1 = b.s1, E = b.esf, nc = b.nc;
+  const int32_t pitch = s1 | 1;
+  const bool row = k < s0;
+  const int32_t kk = row ? k : k - s0;
+  const int32_t es = b.es0 + E * i + k;
+  const float* lp = io.lp + b.c0 + int64_t(nc) * i;
+  float o = 0.f, x = 0.f, l[kAhead];
+  if (on) {
+    const int32_t vs = g.edge_vs0[b.e0 + 2 * i + (row ? 0 : 1)];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) l[u] = lp[min(k + u * E, nc - 1)];
+    o = io.mo[es];
+    x = io.vsum[vs + kk] - o;
+    xs[k] = row ? 0.f + x : x;
+  }
+  wave_lds_fence();
+  if (on) {
+    int32_t p = k / s1, q = k - p * s1;
+    const int32_t dp = E / s1, dq = E - dp * s1;
+    for (int32_t c0 = k; c0 < nc; c0 += kAhead * E) {
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const int32_t c = c0 + u * E;
+        if (c < nc) {
+          sm[p * pitch + q] = (xs[p] + xs[s0 + q]) + clip_lp(l[u]);
+          p += dp;
+          q += dq;
+          if (q >= s1) {
+            q -= s1;
+            ++p;
+          }
+        }
+      }
+      if (c0 + kAhead * E < nc)
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) l[u] = lp[min(c0 + (kAhead + u) * E, nc - 1)];
+    }
+  }
+  wave_lds_fence();
+  float n = 0.f;
+  if (on) {
+    const float* v = sm + (row ? kk * pitch : kk);
+    const int32_t step = row ? 1 : pitch, cnt = row ? s1 : s0;
+    float m = kNegInf;
+#pragma unroll 4
+    for (int32_t j = 0; j < cnt; ++j) m = nmax(m, v[j * step]);
+    float f = m;
+    if (!kT0) {
+      float u = 0.f;
+#pragma unroll 4
+      for (int32_t j = 0; j < cnt; ++j) u += exp_term(v[j * step] - m, t);
+      f = lse_finish(u, m, t);
+    }
+    n = io.d * o + io.omd * (f - x);
+  }
+  wave_lds_fence();
+  if (on) xs[k] = n;
+  wave_lds_fence();
+  if (on) {
+    const float* v = xs + (row ? 0 : s0);
+    const int32_t cnt = row ? s0 : s1;
+    float mx = kNegInf;
+#pragma unroll 4
+    for (int32_t j = 0; j < cnt; ++j) mx = nmax(mx, v[j]);
+    const float r = nmax(n - mx, kMsgNegInf);
+    dl = nmax(dl, fabsf(r - o));
+    io.mn[es] = r;
+  }
+}
+// LDS floats of one such factor: 64 vtof / messages at most, then the
+// summaries (s0 s1 <= 1,024, an odd pitch adds at most one float per row).
+constexpr int kPairWideLds = 64 + 1024 + 64;
+
 // Any Enum factor: config table in `tables` as [nv edge offsets][esf owning
 // edge][nc * nv edge-state offsets]; summaries are recomputed per edge state
 // instead of being stored, so no per-thread arrays are needed.
@@ -1849,9 +1941,33 @@ __device__ __forceinline__ void pos4_var_x(int4 q, const float* m, const float* 
   stv<NS>(out, acc);
 }
 
-// One variable of degree <= kVarChunk (returns for heavier ones).
+// Lane q of kWideVarLanes lanes that sum one variable of many states
+// (Plan::wide_desc) together, its states strided over the lanes: the same
+// sums in the same order as one thread over all states, with the states'
+// loads of an edge in one access.
+constexpr int kWideVarLanes = 16;
+__device__ __forceinline__ void wide_var_sums(const DevGraph& g, int4 d, int32_t q, const float* m,
+                                              const float* ev, float* out) {
+  for (int32_t s = q; s < d.y; s += kWideVarLanes) {
+    const float e = ev[d.x + s];
+    float acc = 0.f;
+    int32_t p = d.z;
+    for (; p + 4 <= d.z + d.w; p += 4) {
+      float x[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] = m[g.var_adj_es[p + u] + s];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc += x[u];
+    }
+    for (; p < d.z + d.w; ++p) acc += m[g.var_adj_es[p] + s];
+    out[d.x + s] = acc + e;
+  }
+}
+
+// One variable of degree <= kVarChunk (returns for heavier ones, and with
+// wide_apart for those wide_var_sums takes).
 __device__ __forceinline__ void var_sums(const DevGraph& g, int32_t v, const float* m,
-                                         const float* ev, float* out) {
+                                         const float* ev, float* out, bool wide_apart = false) {
   if (g.var_pos4) {  // variables of <= 4 edges: one index load
     const int4 q = g.var_pos4[v];
     const int32_t vs0 = g.var_vs0[v];
@@ -1887,7 +2003,7 @@ __device__ __forceinline__ void var_sums(const DevGraph& g, int32_t v, const flo
     light_var_t<2>(g, v, vs0, ns, m, ev, out);
   } else if (ns <= 8) {
     light_var_t<8>(g, v, vs0, ns, m, ev, out);
-  } else {
+  } else if (!wide_apart) {
     for (int32_t s = 0; s < ns; ++s) {
       float a = 0.f;
       for (int32_t p = p0; p < p1; ++p) a += m[g.var_adj_es[p] + s];

@@ -321,7 +321,7 @@ int pgx_graph_create(const pgx_wiring* wiring, pgx_graph** out) {
   int32_t *var_vs0, *var_eptr, *var_adj_es, *edge_es0, *edge_vs0, *fac_e0, *tables, *heavy;
   int32_t *heavy_cptr, *heavy_pofs, *heavy_chunk_var, *heavy_chunk_k, *edge_var, *perm,
       *var_adj_ref, *heavy_gpofs, *vh_group_h, *vh_group_j, *heavy_col, *heavy_row,
-      *heavy_stride, *chunk_desc, *chunk_desc_ref, *col_desc, *row_desc, *heavy_desc;
+      *heavy_stride, *chunk_desc, *chunk_desc_ref, *col_desc, *row_desc, *heavy_desc, *wide_desc;
   Block* blocks;
   Task* tasks;
   if ((rc = up(P.var_vs0, &var_vs0)) || (rc = up(P.var_eptr, &var_eptr)) ||
@@ -337,7 +337,8 @@ int pgx_graph_create(const pgx_wiring* wiring, pgx_graph** out) {
       (rc = up(P.heavy_col_chunks, &heavy_col)) || (rc = up(P.heavy_row_chunks, &heavy_row)) ||
       (rc = up(P.heavy_chunk_stride, &heavy_stride)) || (rc = up(P.chunk_desc, &chunk_desc)) ||
       (rc = up(P.chunk_desc_ref, &chunk_desc_ref)) || (rc = up(P.col_desc, &col_desc)) ||
-      (rc = up(P.row_desc, &row_desc)) || (rc = up(P.heavy_desc, &heavy_desc))) {
+      (rc = up(P.row_desc, &row_desc)) || (rc = up(P.heavy_desc, &heavy_desc)) ||
+      (rc = up(P.wide_desc, &wide_desc))) {
     pgx_graph_destroy(g);
     return rc;
   }
@@ -367,6 +368,8 @@ int pgx_graph_create(const pgx_wiring* wiring, pgx_graph** out) {
   d.col_desc = reinterpret_cast<const int4*>(col_desc);
   d.row_desc = reinterpret_cast<const int4*>(row_desc);
   d.heavy_desc = reinterpret_cast<const int4*>(heavy_desc);
+  d.wide_desc = reinterpret_cast<const int4*>(wide_desc);
+  d.num_wide = int32_t(P.wide_desc.size() / 4);
   g->chunk_desc_ref = reinterpret_cast<const int4*>(chunk_desc_ref);
   {
     std::vector<int32_t> zeros(P.heavy_chunk_stride.size(), 0);
@@ -469,11 +472,16 @@ int pgx_graph_create(const pgx_wiring* wiring, pgx_graph** out) {
         // wavefront each
         const int32_t lanes =
             (b.pad[0] & 4) ? kWideLanes : ((b.pad[0] & (8 | 16)) ? 64 : 1);
+        // (full pairwise tables above 8 x 8, per-phase kernels: one lane per
+        // edge state, 64 / esf factors per wavefront)
+        const bool wide = multi && (b.pad[0] & 32);
         const bool m = multi && b.kind == kEnumBin2;
-        const int32_t per = m ? T.size * kBin2PerThread : T.size / lanes;
+        const int32_t per = wide ? (T.size / 64) * (64 / b.esf)
+                                 : (m ? T.size * kBin2PerThread : T.size / lanes);
+        const int32_t pad =
+            wide ? kPairWideTile : (m ? -kBin2PerThread : (lanes == 1 ? 0 : lanes));
         for (int32_t i0 = 0; i0 < b.count; i0 += per)
-          tiles.push_back(Tile{bi, i0, std::min(b.count, i0 + per),
-                               m ? -kBin2PerThread : (lanes == 1 ? 0 : lanes)});
+          tiles.push_back(Tile{bi, i0, std::min(b.count, i0 + per), pad});
       }
     }
     T.kind_tile0[kTileGroups] = int32_t(tiles.size());

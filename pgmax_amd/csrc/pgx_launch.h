@@ -88,6 +88,7 @@ struct KernelClock {
 constexpr int kPhaseThreads = 256;
 constexpr int32_t kMaxBatchPerLaunch = 65535;  // batch elements index grid dimension y
 constexpr int kTileFactors = 256;
+constexpr int32_t kPairWideTile = -64;  // Tile::pad of tiles run by pair_wide (msets)
 constexpr int32_t kBin2PerThread = 4;  // 2x2 factors per thread in k_fac_phase (msets tiles)
 constexpr int64_t kFusedMaxStates = int64_t(1) << 24;  // untuned fused shape up to this many
                                                        // edge states per run

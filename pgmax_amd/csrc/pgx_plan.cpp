@@ -396,13 +396,17 @@ int build_plan(const pgx_wiring& w, Plan* P, std::string* err, int64_t merge_bel
         b.kind = kEnumGeneral;
         if (nv == 2) {
           const int32_t s0 = P->edge_es0[e0 + 1] - es0, s1 = esf - s0;
-          bool full = info.nc == s0 * s1 && s0 <= 8 && s1 <= 8;
+          bool full = info.nc == int64_t(s0) * s1;
           for (int32_t c = 0; full && !info.full && c < info.nc; ++c)
             full = info.table[2 * c] == c / s1 && info.table[2 * c + 1] == s0 + c % s1;
-          if (full) {
+          if (full && s0 <= 8 && s1 <= 8) {
             b.kind = (s0 == 2 && s1 == 2) ? kEnumBin2 : kEnumPair;
             b.s0 = s0;
             b.s1 = s1;
+          } else if (full && esf <= kPairWideStates) {
+            b.s0 = s0;
+            b.s1 = s1;
+            b.pad[0] = 32;
           }
         }
         if (b.kind == kEnumGeneral) {
@@ -526,6 +530,13 @@ int build_plan(const pgx_wiring& w, Plan* P, std::string* err, int64_t merge_bel
     if (P->edge_es0[e + 1] - P->edge_es0[e] == 2 && (P->edge_es0[e] & 1)) P->even2 = false;
   for (int32_t v = 0; v < NV && P->even2; ++v)
     if (P->var_vs0[v + 1] - P->var_vs0[v] == 2 && (P->var_vs0[v] & 1)) P->even2 = false;
+
+  for (int32_t v = 0; v < NV; ++v) {
+    const int32_t ns = P->var_vs0[v + 1] - P->var_vs0[v];
+    const int32_t deg = P->var_eptr[v + 1] - P->var_eptr[v];
+    if (ns > kThreadStates && deg <= kVarChunk)
+      P->wide_desc.insert(P->wide_desc.end(), {P->var_vs0[v], ns, P->var_eptr[v], deg});
+  }
 
   // position descriptors of low-degree variables
   if (int64_t(NV) * 16 <= kPos4MaxBytes) {

@@ -43,7 +43,9 @@ struct Block {
                    // bit 1: 2x2 block stored planar (see Plan::perm),
                    // bit 2: OR/AND block run by lane groups (wide factors),
                    // bit 3: general Enum block run by one wavefront per factor,
-                   // bit 4: OR/AND block run by one wavefront per factor
+                   // bit 4: OR/AND block run by one wavefront per factor,
+                   // bit 5: general Enum block of full pairwise tables (s0 x s1,
+                   // row-major) run with one lane per edge state (pair_wide)
 };
 
 // Long sums (incident edges of a variable, parents of a logical factor) run
@@ -57,6 +59,12 @@ constexpr int32_t kWaveLogicalParents = 256;  // parents of a logical factor on 
 // summaries and edge-state vtof fit the wavefront's LDS.
 constexpr int32_t kWaveMaxConfigs = 1024;
 constexpr int32_t kWaveMaxStates = 256;
+// Full pairwise tables larger than 8 x 8: one lane per edge state of the
+// factor, 64 / (s0 + s1) factors per wavefront, their summaries in the
+// wavefront's LDS.
+constexpr int32_t kPairWideStates = 64;  // most edge states of such a factor
+// Variables of more than kThreadStates states are summed by a lane group each.
+constexpr int32_t kThreadStates = 8;
 constexpr int64_t kPos4MaxBytes = int64_t(1) << 30;        // per-variable descriptors
 constexpr int64_t kEdgePos4MaxBytes = int64_t(64) << 20;   // per-edge descriptors
 
@@ -112,6 +120,9 @@ struct Plan {
   // Heavy-variable descriptors, 4 ints each: [first variable state,
   // chunks | ns << 16, first chunk slot, first group slot or -1].
   std::vector<int32_t> heavy_desc;
+  // Variables of more than kThreadStates states and at most kVarChunk edges,
+  // 4 ints each: [first variable state, states, first adjacency index, edges].
+  std::vector<int32_t> wide_desc;
   std::vector<int32_t> heavy_col_chunks;
   std::vector<int32_t> heavy_row_chunks;
   std::vector<int32_t> heavy_gpofs;
