@@ -114,6 +114,7 @@ __device__ __forceinline__ void fac_phase_body(const DevGraph& g, const Tile* ti
   const int32_t b = int32_t(by);
   const Tile tile = tiles[bx];
   const Block blk = g.blocks[tile.block];
+  if (task_done(g, r, b, blk.task, it)) return;
   const float* xb = r.x + b * g.num_es;
   const float* yb = r.y + b * g.num_es;
   const float* mo = ((r.n_it - it) & 1) ? yb : xb;
@@ -127,7 +128,7 @@ __device__ __forceinline__ void fac_phase_body(const DevGraph& g, const Tile* ti
       if (i < tile.i1)
         logical_factor_wave<EngineIO>(g, blk.f0 + i, blk.off, io, t, true, dl,
                                       int32_t(threadIdx.x) % 64);
-      block_delta_store<kPhaseThreads>(dl, delta_slot(r, b, it));
+      block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
       return;
     }
     if (tile.pad == kWideLanes) {  // one lane group per factor
@@ -135,7 +136,7 @@ __device__ __forceinline__ void fac_phase_body(const DevGraph& g, const Tile* ti
       if (i < tile.i1)
         logical_factor_wide<EngineIO>(g, blk.f0 + i, blk.off, io, t, true, dl,
                                       int32_t(threadIdx.x) % kWideLanes);
-      block_delta_store<kPhaseThreads>(dl, delta_slot(r, b, it));
+      block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
       return;
     }
   }
@@ -151,14 +152,14 @@ __device__ __forceinline__ void fac_phase_body(const DevGraph& g, const Tile* ti
       float* xs = wl[w] + fl * (blk.esf + blk.s0 * (blk.s1 | 1));
       pair_wide<kT0>(g, blk, i, fl < fw && i < tile.i1, lane - fl * blk.esf, io, t, dl, xs,
                      xs + blk.esf);
-      block_delta_store<kPhaseThreads>(dl, delta_slot(r, b, it));
+      block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
       return;
     }
     if (tile.pad == 64) {  // one wavefront per factor
       const int32_t i = tile.i0 + w;
       enum_general_wave<EngineIO, kT0>(g, blk, i, i < tile.i1, io, t, dl,
                                        int32_t(threadIdx.x) & 63, wl[w], wl[w] + kWaveMaxConfigs);
-      block_delta_store<kPhaseThreads>(dl, delta_slot(r, b, it));
+      block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
       return;
     }
   }
@@ -176,13 +177,13 @@ __device__ __forceinline__ void fac_phase_body(const DevGraph& g, const Tile* ti
         for (int k = 0; k < kBin2PerThread; ++k)
           if (idx[k] >= 0) factor_update<EngineIO, kT0, (1 << KIND)>(g, blk, idx[k], io, t, true, dl);
       }
-      block_delta_store<kPhaseThreads>(dl, delta_slot(r, b, it));
+      block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
       return;
     }
   }
   const int32_t i = tile.i0 + threadIdx.x;
   if (i < tile.i1) factor_update<EngineIO, kT0, (1 << KIND)>(g, blk, i, io, t, true, dl);
-  block_delta_store<kPhaseThreads>(dl, delta_slot(r, b, it));
+  block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
 }
 
 // Square pairwise Enum blocks (S x S, 3 <= S <= 8; the fused form also
@@ -225,6 +226,7 @@ __device__ __forceinline__ void pair_lanes_phase(const DevGraph& g, const Tile* 
   const int32_t b = int32_t(by);
   const Tile tile = tiles[bx];
   const Block blk = g.blocks[tile.block];
+  if (task_done(g, r, b, blk.task, it)) return;
   const float* xb = r.x + b * g.num_es;
   const float* yb = r.y + b * g.num_es;
   const float* mo = ((r.n_it - it) & 1) ? yb : xb;
@@ -257,7 +259,7 @@ __device__ __forceinline__ void pair_lanes_phase(const DevGraph& g, const Tile* 
     case 7: body(std::integral_constant<int, 7>{}); break;
     default: body(std::integral_constant<int, 8>{}); break;
   }
-  block_delta_store<kPhaseThreads>(dl, delta_slot(r, b, it));
+  block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
 }
 
 // Lane-group tile t of batch element b: do all its factors hold the tile's
@@ -324,6 +326,7 @@ __device__ __forceinline__ void fac_fused_body(const DevGraph& g, const Tile* ti
   const int32_t b = blockIdx.y;
   const Tile tile = tiles[blockIdx.x];
   const Block blk = g.blocks[tile.block];
+  if (task_done(g, r, b, blk.task, it)) return;
   const float* xb = r.x + b * g.num_es;
   const float* yb = r.y + b * g.num_es;
   FusedIO io;
@@ -344,7 +347,7 @@ __device__ __forceinline__ void fac_fused_body(const DevGraph& g, const Tile* ti
   float dl = 0.f;
   const int32_t i = tile.i0 + threadIdx.x;
   if (i < tile.i1) fused_factor_update<kT0, KINDS>(g, blk, i, io, t, dl);
-  block_delta_store<kPhaseThreads>(dl, delta_slot(r, b, it));
+  block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
 }
 
 template <bool kT0, int KINDS>
@@ -392,6 +395,45 @@ __global__ void __launch_bounds__(kPhaseThreads)
       block_delta<kPhaseThreads>(dl, r.deltas + b * r.n_it + it);
     }
     grid.sync();
+  }
+}
+
+// Iterations of every (batch element, task) of a per-phase convergence run:
+// up to and including the first whose delta is <= tol, or all n_it. One
+// wavefront each.
+__global__ void __launch_bounds__(64) k_converge_iters(DevGraph g, RunBufs r) {
+  const int32_t ti = blockIdx.x, b = blockIdx.y;
+  int32_t first = r.n_it - 1;
+  for (int32_t it = threadIdx.x; it < first; it += 64)
+    if (*task_delta(g, r, b, ti, it) <= r.tol) first = it;
+  for (int o = 32; o > 0; o >>= 1) first = min(first, __shfl_xor(first, o, 64));
+  if (threadIdx.x == 0) r.iters_done[int64_t(b) * g.num_tasks + ti] = first + 1;
+}
+
+// The messages of a per-phase convergence run: a task that stopped after n
+// iterations left them in the buffer iteration n - 1 wrote, in the engine's
+// layout; out is the reference's (the buffer x itself when the layouts are
+// the same: only tasks that stopped in the other buffer are copied then).
+__global__ void __launch_bounds__(256)
+    k_converge_out(DevGraph g, const Tile* tiles, RunBufs r, float* out) {
+  const int32_t b = blockIdx.y;
+  const Tile tile = tiles[blockIdx.x];
+  const Block blk = g.blocks[tile.block];
+  const int32_t n = r.iters_done[int64_t(b) * g.num_tasks + blk.task];
+  const bool in_y = ((r.n_it - n) & 1) != 0;
+  if (!g.perm && !in_y) return;
+  const float* src = (in_y ? r.y : r.x) + b * g.num_es;
+  float* dst = out + b * g.num_es;
+  const int32_t a = g.edge_es0[g.fac_e0[blk.f0 + tile.i0]];
+  const int32_t z = g.edge_es0[g.fac_e0[blk.f0 + tile.i1]];
+  for (int32_t k = a + int32_t(threadIdx.x); k < z; k += 256) {
+    const int32_t p = g.perm ? g.perm[k] : k;
+    if (g.packed) {
+      const float2 m = pair_decode(src[p >> 1]);
+      dst[k] = (p & 1) ? m.y : m.x;
+    } else {
+      dst[k] = src[p];
+    }
   }
 }
 
@@ -588,6 +630,14 @@ int launch_phased(pgx_graph* g, const RunBufs& r, int32_t batch, hipStream_t s,
   }
   PGX_HIP(hipGetLastError());
   return PGX_OK;
+}
+
+void launch_converge_finish(pgx_graph* g, const RunBufs& r, float* out, int32_t batch,
+                            hipStream_t s) {
+  const TileSet& T = g->tsets[2];
+  hipLaunchKernelGGL(k_converge_iters, dim3(g->dev.num_tasks, batch), dim3(64), 0, s, g->dev, r);
+  hipLaunchKernelGGL(k_converge_out, dim3(T.num_tiles, batch), dim3(256), 0, s, g->dev, T.tiles,
+                     r, out);
 }
 
 template <bool kT0, int KINDS>

@@ -758,6 +758,8 @@ int build_plan(const pgx_wiring& w, Plan* P, std::string* err, int64_t merge_bel
   std::stable_sort(kept.begin(), kept.end(),
                    [](const Task& a, const Task& b) { return a.work > b.work; });
   P->tasks = kept;
+  for (int32_t ti = 0; ti < int32_t(P->tasks.size()); ++ti)
+    for (int32_t bi = P->tasks[ti].b0; bi < P->tasks[ti].b1; ++bi) P->blocks[bi].task = ti;
   return PGX_OK;
 }
 

@@ -27,7 +27,7 @@ enum BlockKind : int32_t {
 
 struct Block {
   int32_t kind;
-  int32_t task;
+  int32_t task;    // index in Plan::tasks
   int32_t f0;      // first factor (global id)
   int32_t count;   // number of factors
   int32_t e0;      // first edge of factor f0

@@ -62,3 +62,51 @@ def test_pairwise_tables_above_8_states(gpu, n0, s0, n1, s1, temperature):
     np.testing.assert_array_equal(_np(deltas), ref_d)
   np.testing.assert_array_equal(_np(bp.context.get_flat_beliefs(out)),
                                 lbp.get_flat_beliefs(g, ref, ev))
+
+
+def _uneven_union(kind):
+  """Connected graphs of different sizes, layouts and factor kinds, and their
+  inputs as one union."""
+  from pgmax_amd import batch
+  rng = np.random.default_rng(5)
+  if kind == "binary":  # one float per message in the per-phase shape
+    ws = [batch.grid_wiring(n, n, 2, torus=True, full_tables=True) for n in (3, 9, 30)]
+  elif kind == "mixed":  # planar and plain blocks, lane-group tiles
+    ws = [batch.grid_wiring(n, n, s, full_tables=True)
+          for n, s in ((2, 2), (7, 5), (20, 2), (3, 8), (12, 3))]
+  elif kind == "heavy":  # stars: centres of 5 and 40 edges, two-kernel iterations
+    ws = [batch.pairwise_wiring(n + 1, s, np.stack([np.zeros(n, int), np.arange(1, n + 1)], 1),
+                                full_tables=True) for n, s in ((5, 3), (40, 2), (40, 4))]
+  else:  # 12 states: general Enum blocks
+    ws = [batch.grid_wiring(n, n, 12, full_tables=True) for n in (2, 5)]
+  bb = batch.BatchedBP(ws, temperature=1.0)
+  lp = rng.normal(0, 0.4, size=bb.layout.num_lp).astype(np.float32)
+  ev = rng.normal(size=bb.layout.num_vs).astype(np.float32)
+  return bb, lp, ev
+
+
+@pytest.mark.parametrize("temperature", [0.0, 1.0])
+@pytest.mark.parametrize("kind", ["binary", "mixed", "heavy", "general"])
+@pytest.mark.parametrize("iters,tol", [(1, 1e-3), (40, 1e-3), (41, 1e-3), (25, 0.0), (7, -1.0),
+                                       (9, 1e30)])
+def test_per_phase_convergence_equals_task_loop(gpu, kind, temperature, iters, tol):
+  """Per-phase convergence runs stop every task where the task loop does, with
+  the same messages, deltas and counts, whichever buffer a task stopped in."""
+  import torch
+  bb, lp, ev = _uneven_union(kind)
+  ft = np.random.default_rng(6).normal(size=bb.layout.num_es).astype(np.float32)
+  got = {}
+  for mode in (1, 2):
+    for fuse in (0, 1):
+      _lib.set_option("mode", mode)
+      _lib.set_option("fuse", fuse)
+      got[mode, fuse] = bb.run_converge(lp, ft, ev, iters, tol, 0.5, temperature)
+  _lib.set_option("mode", 0)
+  got["auto"] = bb.run_converge(lp, ft, ev, iters, tol, 0.5, temperature)
+  ref = got[1, 0]
+  for key, res in got.items():
+    for a, b in zip(res, ref):
+      assert torch.equal(a, b), key
+  n = ref[2].cpu().numpy()
+  assert (n == (1 if tol == 1e30 else iters)).all() or tol in (1e-3, 0.0)
+  bb.close()
