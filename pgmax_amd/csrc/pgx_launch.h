@@ -219,24 +219,26 @@ __device__ __forceinline__ uint32_t* delta_slot(const RunBufs& r, int32_t b, int
   return r.dslot + pair * r.dslot_n + (r.dslot_n > 1 ? int32_t(blockIdx.x) % r.dslot_n : 0);
 }
 
-// Per-phase convergence runs (r.converge): every task of every batch element
-// has its own delta per iteration, zero until a workgroup of the task folds
-// its own into it. A task is done once an iteration's delta is <= tol; its
-// workgroups then leave the later deltas at their initial 0 <= tol, so the
-// previous iteration's delta alone says whether a task is done.
+// Per-phase convergence runs (r.converge; the kernels' kConv instances): every
+// task of every batch element has its own delta per iteration, zero until a
+// workgroup of the task folds its own into it. A task is done once an
+// iteration's delta is <= tol; its workgroups then leave the later deltas at
+// their initial 0 <= tol, so the previous iteration's delta alone says
+// whether a task is done.
 __device__ __forceinline__ float* task_delta(const DevGraph& g, const RunBufs& r, int32_t b,
                                              int32_t task, int32_t it) {
   return r.task_deltas + (int64_t(b) * g.num_tasks + task) * r.n_it + it;
 }
 __device__ __forceinline__ bool task_done(const DevGraph& g, const RunBufs& r, int32_t b,
                                           int32_t task, int32_t it) {
-  return r.converge && it > 0 && *task_delta(g, r, b, task, it - 1) <= r.tol;
+  return it > 0 && *task_delta(g, r, b, task, it - 1) <= r.tol;
 }
 // Where a workgroup of block blk folds its delta.
+template <bool kConv>
 __device__ __forceinline__ uint32_t* delta_dst(const DevGraph& g, const RunBufs& r,
                                                const Block& blk, int32_t b, int32_t it) {
-  return r.converge ? reinterpret_cast<uint32_t*>(task_delta(g, r, b, blk.task, it))
-                    : delta_slot(r, b, it);
+  return kConv ? reinterpret_cast<uint32_t*>(task_delta(g, r, b, blk.task, it))
+               : delta_slot(r, b, it);
 }
 
 struct Tile {

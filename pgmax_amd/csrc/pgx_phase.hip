@@ -106,7 +106,7 @@ __global__ void __launch_bounds__(kPhaseThreads)
 }
 
 // Phased shape: factor phase over tiles of <= kTileFactors factors.
-template <bool kT0, int KIND>
+template <bool kT0, int KIND, bool kConv>
 __device__ __forceinline__ void fac_phase_body(const DevGraph& g, const Tile* tiles,
                                                const RunBufs& r, int32_t it, float t) {
   uint32_t bx, by;
@@ -114,7 +114,7 @@ __device__ __forceinline__ void fac_phase_body(const DevGraph& g, const Tile* ti
   const int32_t b = int32_t(by);
   const Tile tile = tiles[bx];
   const Block blk = g.blocks[tile.block];
-  if (task_done(g, r, b, blk.task, it)) return;
+  if (kConv && task_done(g, r, b, blk.task, it)) return;
   const float* xb = r.x + b * g.num_es;
   const float* yb = r.y + b * g.num_es;
   const float* mo = ((r.n_it - it) & 1) ? yb : xb;
@@ -128,7 +128,7 @@ __device__ __forceinline__ void fac_phase_body(const DevGraph& g, const Tile* ti
       if (i < tile.i1)
         logical_factor_wave<EngineIO>(g, blk.f0 + i, blk.off, io, t, true, dl,
                                       int32_t(threadIdx.x) % 64);
-      block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
+      block_delta_store<kPhaseThreads>(dl, delta_dst<kConv>(g, r, blk, b, it));
       return;
     }
     if (tile.pad == kWideLanes) {  // one lane group per factor
@@ -136,7 +136,7 @@ __device__ __forceinline__ void fac_phase_body(const DevGraph& g, const Tile* ti
       if (i < tile.i1)
         logical_factor_wide<EngineIO>(g, blk.f0 + i, blk.off, io, t, true, dl,
                                       int32_t(threadIdx.x) % kWideLanes);
-      block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
+      block_delta_store<kPhaseThreads>(dl, delta_dst<kConv>(g, r, blk, b, it));
       return;
     }
   }
@@ -152,14 +152,14 @@ __device__ __forceinline__ void fac_phase_body(const DevGraph& g, const Tile* ti
       float* xs = wl[w] + fl * (blk.esf + blk.s0 * (blk.s1 | 1));
       pair_wide<kT0>(g, blk, i, fl < fw && i < tile.i1, lane - fl * blk.esf, io, t, dl, xs,
                      xs + blk.esf);
-      block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
+      block_delta_store<kPhaseThreads>(dl, delta_dst<kConv>(g, r, blk, b, it));
       return;
     }
     if (tile.pad == 64) {  // one wavefront per factor
       const int32_t i = tile.i0 + w;
       enum_general_wave<EngineIO, kT0>(g, blk, i, i < tile.i1, io, t, dl,
                                        int32_t(threadIdx.x) & 63, wl[w], wl[w] + kWaveMaxConfigs);
-      block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
+      block_delta_store<kPhaseThreads>(dl, delta_dst<kConv>(g, r, blk, b, it));
       return;
     }
   }
@@ -177,13 +177,13 @@ __device__ __forceinline__ void fac_phase_body(const DevGraph& g, const Tile* ti
         for (int k = 0; k < kBin2PerThread; ++k)
           if (idx[k] >= 0) factor_update<EngineIO, kT0, (1 << KIND)>(g, blk, idx[k], io, t, true, dl);
       }
-      block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
+      block_delta_store<kPhaseThreads>(dl, delta_dst<kConv>(g, r, blk, b, it));
       return;
     }
   }
   const int32_t i = tile.i0 + threadIdx.x;
   if (i < tile.i1) factor_update<EngineIO, kT0, (1 << KIND)>(g, blk, i, io, t, true, dl);
-  block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
+  block_delta_store<kPhaseThreads>(dl, delta_dst<kConv>(g, r, blk, b, it));
 }
 
 // Square pairwise Enum blocks (S x S, 3 <= S <= 8; the fused form also
@@ -217,7 +217,7 @@ __device__ __forceinline__ void pair_lanes_body(const L& ld, const Tile& tile, c
 
 // kFused: variable sums formed on the factor side (PairFusedLoader, no
 // variable phase); else read from the variable phase's sums.
-template <bool kT0, bool kFused>
+template <bool kT0, bool kFused, bool kConv>
 __device__ __forceinline__ void pair_lanes_phase(const DevGraph& g, const Tile* tiles,
                                                  const RunBufs& r, int32_t it, float t) {
   __shared__ float lds[kPhaseThreads / 64][kPairLanesLds];
@@ -226,7 +226,7 @@ __device__ __forceinline__ void pair_lanes_phase(const DevGraph& g, const Tile* 
   const int32_t b = int32_t(by);
   const Tile tile = tiles[bx];
   const Block blk = g.blocks[tile.block];
-  if (task_done(g, r, b, blk.task, it)) return;
+  if (kConv && task_done(g, r, b, blk.task, it)) return;
   const float* xb = r.x + b * g.num_es;
   const float* yb = r.y + b * g.num_es;
   const float* mo = ((r.n_it - it) & 1) ? yb : xb;
@@ -259,7 +259,7 @@ __device__ __forceinline__ void pair_lanes_phase(const DevGraph& g, const Tile* 
     case 7: body(std::integral_constant<int, 7>{}); break;
     default: body(std::integral_constant<int, 8>{}); break;
   }
-  block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
+  block_delta_store<kPhaseThreads>(dl, delta_dst<kConv>(g, r, blk, b, it));
 }
 
 // Lane-group tile t of batch element b: do all its factors hold the tile's
@@ -290,43 +290,43 @@ __global__ void __launch_bounds__(256)
   if (threadIdx.x == 0) share[int64_t(b) * num_tiles + t] = same;
 }
 
-template <bool kT0>
+template <bool kT0, bool kConv>
 __global__ void __launch_bounds__(kPhaseThreads)
     k_pair_lanes(DevGraph g, const Tile* tiles, RunBufs r, int32_t it) {
   if (!kT0 && r.t == 1.f)
-    pair_lanes_phase<kT0, false>(g, tiles, r, it, 1.f);
+    pair_lanes_phase<kT0, false, kConv>(g, tiles, r, it, 1.f);
   else
-    pair_lanes_phase<kT0, false>(g, tiles, r, it, r.t);
+    pair_lanes_phase<kT0, false, kConv>(g, tiles, r, it, r.t);
 }
 
 // The whole iteration of a graph of 2 x 2 and square pairwise blocks whose
 // variables have at most 4 edges, in one launch (no variable phase).
-template <bool kT0>
+template <bool kT0, bool kConv>
 __global__ void __launch_bounds__(kPhaseThreads)
     k_pair_lanes_fused(DevGraph g, const Tile* tiles, RunBufs r, int32_t it) {
   if (!kT0 && r.t == 1.f)
-    pair_lanes_phase<kT0, true>(g, tiles, r, it, 1.f);
+    pair_lanes_phase<kT0, true, kConv>(g, tiles, r, it, 1.f);
   else
-    pair_lanes_phase<kT0, true>(g, tiles, r, it, r.t);
+    pair_lanes_phase<kT0, true, kConv>(g, tiles, r, it, r.t);
 }
 
-template <bool kT0, int KIND>
+template <bool kT0, int KIND, bool kConv>
 __global__ void __launch_bounds__(kPhaseThreads)
     k_fac_phase(DevGraph g, const Tile* tiles, RunBufs r, int32_t it) {
   if (!kT0 && r.t == 1.f)
-    fac_phase_body<kT0, KIND>(g, tiles, r, it, 1.f);
+    fac_phase_body<kT0, KIND, kConv>(g, tiles, r, it, 1.f);
   else
-    fac_phase_body<kT0, KIND>(g, tiles, r, it, r.t);
+    fac_phase_body<kT0, KIND, kConv>(g, tiles, r, it, r.t);
 }
 
 // Phased shape for fusable graphs: the whole iteration in one launch.
-template <bool kT0, int KINDS>
+template <bool kT0, int KINDS, bool kConv>
 __device__ __forceinline__ void fac_fused_body(const DevGraph& g, const Tile* tiles,
                                                const RunBufs& r, int32_t it, float t) {
   const int32_t b = blockIdx.y;
   const Tile tile = tiles[blockIdx.x];
   const Block blk = g.blocks[tile.block];
-  if (task_done(g, r, b, blk.task, it)) return;
+  if (kConv && task_done(g, r, b, blk.task, it)) return;
   const float* xb = r.x + b * g.num_es;
   const float* yb = r.y + b * g.num_es;
   FusedIO io;
@@ -347,16 +347,16 @@ __device__ __forceinline__ void fac_fused_body(const DevGraph& g, const Tile* ti
   float dl = 0.f;
   const int32_t i = tile.i0 + threadIdx.x;
   if (i < tile.i1) fused_factor_update<kT0, KINDS>(g, blk, i, io, t, dl);
-  block_delta_store<kPhaseThreads>(dl, delta_dst(g, r, blk, b, it));
+  block_delta_store<kPhaseThreads>(dl, delta_dst<kConv>(g, r, blk, b, it));
 }
 
-template <bool kT0, int KINDS>
+template <bool kT0, int KINDS, bool kConv>
 __global__ void __launch_bounds__(kPhaseThreads)
     k_fac_fused(DevGraph g, const Tile* tiles, RunBufs r, int32_t it) {
   if (!kT0 && r.t == 1.f)
-    fac_fused_body<kT0, KINDS>(g, tiles, r, it, 1.f);
+    fac_fused_body<kT0, KINDS, kConv>(g, tiles, r, it, 1.f);
   else
-    fac_fused_body<kT0, KINDS>(g, tiles, r, it, r.t);
+    fac_fused_body<kT0, KINDS, kConv>(g, tiles, r, it, r.t);
 }
 
 // Cooperative shape for fusable graphs: every iteration in one launch of
@@ -514,7 +514,7 @@ void launch_pair_unpack(const DevGraph& d, const float* packed, int64_t stride, 
   hipLaunchKernelGGL(k_pair_unpack, ugrid, dim3(256), 0, s, d, packed, stride, out);
 }
 
-template <bool kT0>
+template <bool kT0, bool kConv>
 static void launch_fac_kinds(pgx_graph* g, const TileSet& T, const RunBufs& r, int32_t batch,
                              int32_t it, hipStream_t s, const KernelClock& clk, bool lanes) {
   const DevGraph& d = g->dev;
@@ -523,28 +523,28 @@ static void launch_fac_kinds(pgx_graph* g, const TileSet& T, const RunBufs& r, i
   const dim3 blk(T.size);
   const int32_t id0 = PGX_KERNEL_FAC_PHASE;
   if (k0[1] > k0[0])
-    clk.run(id0 + 0, [&] { hipLaunchKernelGGL((k_fac_phase<kT0, 0>), grid(0), blk, 0, s, d, T.tiles + k0[0], r, it); });
+    clk.run(id0 + 0, [&] { hipLaunchKernelGGL((k_fac_phase<kT0, 0, kConv>), grid(0), blk, 0, s, d, T.tiles + k0[0], r, it); });
   if (k0[2] > k0[1])
-    clk.run(id0 + 1, [&] { hipLaunchKernelGGL((k_fac_phase<kT0, 1>), grid(1), blk, 0, s, d, T.tiles + k0[1], r, it); });
+    clk.run(id0 + 1, [&] { hipLaunchKernelGGL((k_fac_phase<kT0, 1, kConv>), grid(1), blk, 0, s, d, T.tiles + k0[1], r, it); });
   if (k0[3] > k0[2])
-    clk.run(id0 + 2, [&] { hipLaunchKernelGGL((k_fac_phase<kT0, 2>), grid(2), blk, 0, s, d, T.tiles + k0[2], r, it); });
+    clk.run(id0 + 2, [&] { hipLaunchKernelGGL((k_fac_phase<kT0, 2, kConv>), grid(2), blk, 0, s, d, T.tiles + k0[2], r, it); });
   if (k0[4] > k0[3])
-    clk.run(id0 + 3, [&] { hipLaunchKernelGGL((k_fac_phase<kT0, 3>), grid(3), blk, 0, s, d, T.tiles + k0[3], r, it); });
+    clk.run(id0 + 3, [&] { hipLaunchKernelGGL((k_fac_phase<kT0, 3, kConv>), grid(3), blk, 0, s, d, T.tiles + k0[3], r, it); });
   if (k0[5] > k0[4])
-    clk.run(id0 + 4, [&] { hipLaunchKernelGGL((k_fac_phase<kT0, 4>), grid(4), blk, 0, s, d, T.tiles + k0[4], r, it); });
+    clk.run(id0 + 4, [&] { hipLaunchKernelGGL((k_fac_phase<kT0, 4, kConv>), grid(4), blk, 0, s, d, T.tiles + k0[4], r, it); });
   if (k0[6] > k0[5])
-    clk.run(id0 + 5, [&] { hipLaunchKernelGGL((k_fac_phase<kT0, 5>), grid(5), blk, 0, s, d, T.tiles + k0[5], r, it); });
+    clk.run(id0 + 5, [&] { hipLaunchKernelGGL((k_fac_phase<kT0, 5, kConv>), grid(5), blk, 0, s, d, T.tiles + k0[5], r, it); });
   // square pairwise blocks on lane groups or one factor per thread (timed
   // as the pairwise Enum kind)
   constexpr int kL = kPairLanesGroup, kT = kPairThreadGroup;
   if (lanes && k0[kL + 1] > k0[kL])
     clk.run(id0 + kEnumPair, [&] {
-      hipLaunchKernelGGL((k_pair_lanes<kT0>), grid(kL), dim3(kPhaseThreads), 0, s, d,
+      hipLaunchKernelGGL((k_pair_lanes<kT0, kConv>), grid(kL), dim3(kPhaseThreads), 0, s, d,
                          T.tiles + k0[kL], r, it);
     });
   if (!lanes && k0[kT + 1] > k0[kT])
     clk.run(id0 + kEnumPair, [&] {
-      hipLaunchKernelGGL((k_fac_phase<kT0, kEnumPair>), grid(kT), blk, 0, s, d, T.tiles + k0[kT],
+      hipLaunchKernelGGL((k_fac_phase<kT0, kEnumPair, kConv>), grid(kT), blk, 0, s, d, T.tiles + k0[kT],
                          r, it);
     });
 }
@@ -566,8 +566,8 @@ static RunBufs with_shared_tables(const DevGraph& d, const Tile* tiles, int32_t 
   return rr;
 }
 
-template <bool kT0>
-int launch_phased(pgx_graph* g, const RunBufs& r, int32_t batch, hipStream_t s,
+template <bool kT0, bool kConv>
+static int launch_phased_t(pgx_graph* g, const RunBufs& r, int32_t batch, hipStream_t s,
                   const KernelClock& clk, int64_t tile, int64_t threads, bool lanes) {
   const DevGraph& d = g->dev;
   const TileSet& T = g->tsets[tile <= 64 ? 0 : (tile <= 128 ? 1 : 2)];
@@ -597,7 +597,7 @@ int launch_phased(pgx_graph* g, const RunBufs& r, int32_t batch, hipStream_t s,
     const RunBufs rr = with_shared_tables(d, L.tiles, L.num_tiles, r, batch, s);
     for (int32_t it = 0; it < rr.n_it; ++it)
       clk.run(PGX_KERNEL_FAC_FUSED, [&] {
-        hipLaunchKernelGGL((k_pair_lanes_fused<kT0>), lgrid, dim3(kPhaseThreads), 0, s, d,
+        hipLaunchKernelGGL((k_pair_lanes_fused<kT0, kConv>), lgrid, dim3(kPhaseThreads), 0, s, d,
                            L.tiles, rr, it);
       });
     PGX_HIP(hipGetLastError());
@@ -607,10 +607,10 @@ int launch_phased(pgx_graph* g, const RunBufs& r, int32_t batch, hipStream_t s,
     for (int32_t it = 0; it < r.n_it; ++it) {
       clk.run(PGX_KERNEL_FAC_FUSED, [&] {
         if (g->kinds_mask == kKindsBin2)
-          hipLaunchKernelGGL((k_fac_fused<kT0, kKindsBin2>), fgrid, dim3(T.size), 0, s, d,
+          hipLaunchKernelGGL((k_fac_fused<kT0, kKindsBin2, kConv>), fgrid, dim3(T.size), 0, s, d,
                              T.tiles, r, it);
         else
-          hipLaunchKernelGGL((k_fac_fused<kT0, kKindsPairwise>), fgrid, dim3(T.size), 0, s,
+          hipLaunchKernelGGL((k_fac_fused<kT0, kKindsPairwise, kConv>), fgrid, dim3(T.size), 0, s,
                              d, T.tiles, r, it);
       });
     }
@@ -626,10 +626,17 @@ int launch_phased(pgx_graph* g, const RunBufs& r, int32_t batch, hipStream_t s,
     if (d.num_vars > 0)
       launch_var_phase(d, mo, d.num_es, rr.ev, rr.ev_stride, rr.vsum, rr.partial, batch, s, &clk,
                        rr.xcd);
-    launch_fac_kinds<kT0>(g, M, rr, batch, it, s, clk, lanes);
+    launch_fac_kinds<kT0, kConv>(g, M, rr, batch, it, s, clk, lanes);
   }
   PGX_HIP(hipGetLastError());
   return PGX_OK;
+}
+
+template <bool kT0>
+int launch_phased(pgx_graph* g, const RunBufs& r, int32_t batch, hipStream_t s,
+                  const KernelClock& clk, int64_t tile, int64_t threads, bool lanes) {
+  return r.converge ? launch_phased_t<kT0, true>(g, r, batch, s, clk, tile, threads, lanes)
+                    : launch_phased_t<kT0, false>(g, r, batch, s, clk, tile, threads, lanes);
 }
 
 void launch_converge_finish(pgx_graph* g, const RunBufs& r, float* out, int32_t batch,
