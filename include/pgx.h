@@ -295,7 +295,8 @@ int pgx_enum_rows_fac_to_var(const int32_t* cfg_row_ptr, const int32_t* row_es,
  * and replays it on later calls with the same arguments; at most 8 graphs
  * per pgx_graph, freed with it; default 0),
  * "tile" (factors and threads per workgroup of the per-phase factor
- * kernels: 64, 128 or 256; columns per 32-row tile of the complete
+ * kernels: 64, 128 or 256; lane-group tiles of small graphs also 16 and 32,
+ * one and two passes; columns per 32-row tile of the complete
  * bipartite iteration: 32, 64 or 128; 0 auto), "planar" (read by pgx_graph_create: 1,
  * the default, stores the messages of each block of 2x2 Enum factors as two
  * planes, first edges then second edges, inside the engine; results are

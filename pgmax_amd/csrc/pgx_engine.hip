@@ -496,9 +496,9 @@ int pgx_graph_create(const pgx_wiring* wiring, pgx_graph** out) {
   bool lane_fusable = !P.blocks.empty() && !P.var_pos4.empty() && P.max_degree <= 4;
   for (const Block& b : P.blocks)
     lane_fusable = lane_fusable && (b.kind == kEnumBin2 || lane_pair(b));
-  for (int ts = 0; ts < 3 && lane_fusable; ++ts) {
+  for (int ts = 0; ts < kLaneSets && lane_fusable; ++ts) {
     TileSet& T = g->lsets[ts];
-    T.size = kTileSizes[ts];
+    T.size = kPhaseThreads;
     std::vector<Tile> tiles;
     for (int32_t bi = 0; bi < int32_t(P.blocks.size()); ++bi) {
       const Block& b = P.blocks[bi];
@@ -647,13 +647,45 @@ static int32_t delta_slots(const pgx_graph* g, int32_t batch, int32_t n_it) {
   return n;
 }
 
+// Lane-group tile sets a run of `batch` elements may use: those of 1 and 2
+// passes only where the 1-pass tiles are at most kSmallLaneTiles, which keeps
+// the scratch of larger runs (share_bytes) what 4-pass tiles need.
+constexpr int64_t kSmallLaneTiles = 4096;
+static int lane_sets_from(const pgx_graph* g, int32_t batch) {
+  return int64_t(g->lsets[0].num_tiles) * batch <= kSmallLaneTiles ? 0 : 2;
+}
+// The set for a "tile" option of 16, 32, 64, 128, 256; untuned (0) the one of
+// most passes that still leaves enough workgroups. A tile's passes follow each
+// other, so where the chip is not full they are its time (a 30 x 30 grid of 5
+// states, us an iteration: 16 passes 19.3, 8 11.7, 4 8.2, 2 6.1, 1 5.3); with
+// more workgroups than the CUs hold, more passes pipeline their loads and
+// share one table row (64 Potts grids up to 110 x 110 x 8: 1,867 workgroups of
+// 8 passes 49.1, 14,719 of one 55.7), and many short ones cost their start
+// (64 grids up to 30 x 30: 636 of 2 passes 12.0, 1,236 of one 15.3). 16 passes
+// only pay past what the CUs hold twice (384 grids up to 40 x 40: 830 of 16
+// 50.6, 1,438 of 8 40.0; 256 grids up to 128 x 128: 4,438 of 16 220.9, 8,738 of
+// 8 230.0). Convergence runs lose workgroups as graphs finish, so they take
+// four times as many (the 384 grids: 2,666 of 4 passes 24.6, 1,438 of 8 28.1).
+static int lane_set(const pgx_graph* g, int32_t batch, int64_t tile, bool converge) {
+  const int lo = lane_sets_from(g, batch);
+  if (tile > 0)
+    return std::max(lo, tile <= 16 ? 0 : tile <= 32 ? 1 : tile <= 64 ? 2 : tile <= 128 ? 3 : 4);
+  int ls = kLaneSets - 1;
+  for (; ls > lo; --ls) {
+    const int64_t least = ls == kLaneSets - 1 ? 4096 : (converge ? 2400 : 600);
+    if (int64_t(g->lsets[ls].num_tiles) * batch >= least) break;
+  }
+  return ls;
+}
+
 // Flags of the lane tiles (RunBufs::share), for the largest lane group of
 // the three tile sets and the largest set of fused lane tiles.
 static size_t share_bytes(const pgx_graph* g, int32_t batch) {
   int64_t n = 0;
   for (const TileSet& T : g->msets)
     n = std::max<int64_t>(n, T.kind_tile0[kPairLanesGroup + 1] - T.kind_tile0[kPairLanesGroup]);
-  for (const TileSet& T : g->lsets) n = std::max<int64_t>(n, T.num_tiles);
+  for (int ls = lane_sets_from(g, batch); ls < kLaneSets; ++ls)
+    n = std::max<int64_t>(n, g->lsets[ls].num_tiles);
   return size_t(batch) * size_t(n) * sizeof(int32_t);
 }
 
@@ -792,6 +824,7 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
       chosen = true;
     }
   }
+  const int lset = lane_set(g, batch, tile, converge);
   if (tile == 0) tile = 256;
   r.xcd = int32_t(std::max<int64_t>(0, std::min<int64_t>(xcd, 1024)));
   const bool small_run = int64_t(batch) * d.num_es <= kFusedMaxStates;
@@ -866,8 +899,8 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
     // reading shared tables pays when the one pass that finds them is short
     // next to the run (it reads every table once)
     if (!(share && n_it >= 8)) r.share_mem = nullptr;
-    rc = t0 ? launch_phased<true>(g, r, batch, s, clk, tile, bs, lanes != 0)
-            : launch_phased<false>(g, r, batch, s, clk, tile, bs, lanes != 0);
+    rc = t0 ? launch_phased<true>(g, r, batch, s, clk, tile, bs, lanes != 0, lset)
+            : launch_phased<false>(g, r, batch, s, clk, tile, bs, lanes != 0, lset);
     if (rc == PGX_OK && r.dslot_n > 1) {  // the per-launch kernels wrote delta slots
       const int64_t nd = int64_t(batch) * n_it;
       hipLaunchKernelGGL(k_delta_reduce, dim3(std::min<int64_t>((nd + 255) / 256, 1024)),
@@ -1110,6 +1143,8 @@ int pgx_autotune(pgx_graph* g, const float* lp, int64_t lp_stride, const float* 
           for (int64_t ln : {1, 0}) cands.push_back(RunCfg{2, 0, 0, 3, 256, ln, x});
       // fused lane groups: also one factor per thread, and XCD runs
       if (fuse_opts[fi] && g->lsets[0].num_tiles > 0) {
+        if (lane_sets_from(g, batch) == 0)
+          for (int64_t t : {16, 32}) cands.push_back(RunCfg{2, 0, 1, 3, t});
         cands.push_back(RunCfg{2, 0, 1, 3, 256, 0, 0});
         for (int64_t x : {4, 16}) cands.push_back(RunCfg{2, 0, 1, 3, 256, 1, x});
       }

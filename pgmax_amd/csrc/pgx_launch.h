@@ -267,7 +267,8 @@ struct TileSet {
   int32_t size = 256;
 };
 constexpr int kTileSizes[3] = {64, 128, 256};
-constexpr int kLaneFusedPasses[3] = {4, 8, 16};
+constexpr int kLaneSets = 5;  // lane-group tile sets: passes per wavefront of a tile
+constexpr int kLaneFusedPasses[kLaneSets] = {1, 2, 4, 8, 16};
 
 constexpr int kBipRows = kVarChunk;  // rows per tile of k_bipartite: one column chunk
 
@@ -290,9 +291,8 @@ struct pgx_graph {
   pgx::TileSet msets[3];  // the same with kBin2PerThread 2x2 factors per thread
   // lane-group tiles of every block, for graphs of 2 x 2 and square pairwise
   // blocks whose variables have at most 4 edges (k_pair_lanes_fused; empty
-  // otherwise), with kLaneFusedPasses passes per wavefront (tile option 64,
-  // 128, 256 -> 4, 8, 16)
-  pgx::TileSet lsets[3];
+  // otherwise), with kLaneFusedPasses passes per wavefront (lane_set)
+  pgx::TileSet lsets[pgx::kLaneSets];
   // shapes chosen by pgx_autotune, keyed by (batch, temperature == 0, converge)
   std::map<std::tuple<int32_t, int, int>, pgx::RunCfg> tuned;
   // runs captured as HIP graphs (option "graph"), keyed by every launch argument
@@ -324,7 +324,8 @@ void launch_var_phase(const DevGraph& d, const float* m, int64_t m_stride, const
                       hipStream_t s, const KernelClock* clk = nullptr, int32_t xcd = 0);
 template <bool kT0>
 int launch_phased(pgx_graph* g, const RunBufs& r, int32_t batch, hipStream_t s,
-                  const KernelClock& clk, int64_t tile, int64_t threads, bool lanes);
+                  const KernelClock& clk, int64_t tile, int64_t threads, bool lanes,
+                  int lane_set);
 // After the launches of a per-phase convergence run: iteration counts of every
 // task and the messages of exactly that many iterations into out.
 void launch_converge_finish(pgx_graph* g, const RunBufs& r, float* out, int32_t batch,

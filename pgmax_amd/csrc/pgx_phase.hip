@@ -568,7 +568,7 @@ static RunBufs with_shared_tables(const DevGraph& d, const Tile* tiles, int32_t 
 
 template <bool kT0, bool kConv>
 static int launch_phased_t(pgx_graph* g, const RunBufs& r, int32_t batch, hipStream_t s,
-                  const KernelClock& clk, int64_t tile, int64_t threads, bool lanes) {
+                  const KernelClock& clk, int64_t tile, int64_t threads, bool lanes, int lane_set) {
   const DevGraph& d = g->dev;
   const TileSet& T = g->tsets[tile <= 64 ? 0 : (tile <= 128 ? 1 : 2)];
   const dim3 fgrid(T.num_tiles, batch);
@@ -592,7 +592,7 @@ static int launch_phased_t(pgx_graph* g, const RunBufs& r, int32_t batch, hipStr
     return PGX_OK;
   }
   if (d.fusable && lanes && !d.packed && g->lsets[0].num_tiles > 0) {
-    const TileSet& L = g->lsets[tile <= 64 ? 0 : (tile <= 128 ? 1 : 2)];
+    const TileSet& L = g->lsets[lane_set];
     const dim3 lgrid(L.num_tiles, batch);
     const RunBufs rr = with_shared_tables(d, L.tiles, L.num_tiles, r, batch, s);
     for (int32_t it = 0; it < rr.n_it; ++it)
@@ -634,9 +634,9 @@ static int launch_phased_t(pgx_graph* g, const RunBufs& r, int32_t batch, hipStr
 
 template <bool kT0>
 int launch_phased(pgx_graph* g, const RunBufs& r, int32_t batch, hipStream_t s,
-                  const KernelClock& clk, int64_t tile, int64_t threads, bool lanes) {
-  return r.converge ? launch_phased_t<kT0, true>(g, r, batch, s, clk, tile, threads, lanes)
-                    : launch_phased_t<kT0, false>(g, r, batch, s, clk, tile, threads, lanes);
+                  const KernelClock& clk, int64_t tile, int64_t threads, bool lanes, int lane_set) {
+  return r.converge ? launch_phased_t<kT0, true>(g, r, batch, s, clk, tile, threads, lanes, lane_set)
+                    : launch_phased_t<kT0, false>(g, r, batch, s, clk, tile, threads, lanes, lane_set);
 }
 
 void launch_converge_finish(pgx_graph* g, const RunBufs& r, float* out, int32_t batch,
@@ -710,9 +710,9 @@ int launch_fac_op(pgx_graph* g, int kind, const float* vtof, const float* lp, fl
 }
 
 template int launch_phased<true>(pgx_graph*, const RunBufs&, int32_t, hipStream_t,
-                                 const KernelClock&, int64_t, int64_t, bool);
+                                 const KernelClock&, int64_t, int64_t, bool, int);
 template int launch_phased<false>(pgx_graph*, const RunBufs&, int32_t, hipStream_t,
-                                  const KernelClock&, int64_t, int64_t, bool);
+                                  const KernelClock&, int64_t, int64_t, bool, int);
 template int launch_coop<true>(pgx_graph*, const RunBufs&, int32_t, hipStream_t, int64_t);
 template int launch_coop<false>(pgx_graph*, const RunBufs&, int32_t, hipStream_t, int64_t);
 

@@ -110,3 +110,32 @@ def test_per_phase_convergence_equals_task_loop(gpu, kind, temperature, iters, t
   n = ref[2].cpu().numpy()
   assert (n == (1 if tol == 1e30 else iters)).all() or tol in (1e-3, 0.0)
   bb.close()
+
+
+@pytest.mark.parametrize("tile", [0, 16, 32])
+@pytest.mark.parametrize("temperature", [0.0, 1.0])
+def test_short_lane_tiles_match_oracle(gpu, tile, temperature):
+  """Lane-group tiles of one and two passes (and the untuned choice) on grids
+  whose factors fill no tile, exactly one, and one and a bit, with shared and
+  with own tables."""
+  from pgmax_amd import batch
+  # 64 / S factors per wavefront and pass, four wavefronts: 256 / S a tile
+  ws = [batch.grid_wiring(h, w, s, full_tables=True)
+        for h, w, s in ((2, 2, 3), (1, 33, 8), (1, 34, 8), (1, 49, 5), (1, 50, 5), (9, 13, 2),
+                        (6, 7, 7), (17, 16, 4))]
+  bb = batch.BatchedBP(ws, temperature=temperature)
+  rng = np.random.default_rng(3)
+  shared = np.concatenate([np.tile(rng.normal(size=s * s), nf) for nf, s in (
+      (4, 3), (32, 8), (33, 8), (48, 5), (49, 5), (9 * 12 + 8 * 13, 2), (71, 7), (511, 4))])
+  own = rng.normal(size=shared.size)
+  ev = rng.normal(size=bb.layout.num_vs).astype(np.float32)
+  ft = rng.normal(size=bb.layout.num_es).astype(np.float32)
+  _lib.set_option("tile", tile)
+  for lp in (shared.astype(np.float32), own.astype(np.float32)):
+    assert lp.size == bb.layout.num_lp
+    out, d = bb.run(lp, ft, ev, 9, 0.5, temperature)
+    ref, ref_d = lbp.run_with_diffs(lbp.graph_from_flat(bb.union), lp, ft, ev, 9, 0.5,
+                                    temperature)
+    np.testing.assert_array_equal(_np(out), ref)
+    np.testing.assert_array_equal(_np(d), ref_d)
+  bb.close()
