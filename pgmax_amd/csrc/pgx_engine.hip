@@ -824,10 +824,18 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
       chosen = true;
     }
   }
+  const bool small_run =
+      int64_t(batch) * d.num_es <= (g->kinds_mask == kKindsBin2 ? kFusedMaxBin2 : kFusedMaxStates);
   const int lset = lane_set(g, batch, tile, converge);
-  if (tile == 0) tile = 256;
+  // (two-kernel iterations of 2x2 graphs up to 2^22 edge states, 4 factors per
+  // thread: 16 tori of 128 x 128 14.7 us an iteration in tiles of 256, 13.8 of
+  // 128; 32 of them 21.0 and 21.7)
+  if (tile == 0)
+    tile = (!small_run && g->kinds_mask == kKindsBin2 && !g->bip_plan &&
+            int64_t(batch) * d.num_es <= (int64_t(1) << 22))
+               ? 128
+               : 256;
   r.xcd = int32_t(std::max<int64_t>(0, std::min<int64_t>(xcd, 1024)));
-  const bool small_run = int64_t(batch) * d.num_es <= kFusedMaxStates;
   // k_bipartite numbers (tile, batch element) pairs in one grid dimension
   const int64_t bip_units = int64_t((d.bip_na + d.bip_unary + kBipRows - 1) / kBipRows) *
                             ((d.bip_nb + d.bip_unary + kVarChunk - 1) / kVarChunk) * batch;
@@ -855,8 +863,8 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
   if (bs == 0) bs = 256;
   // Untuned, the per-phase shape recomputes variable sums on the factor side
   // (one launch per iteration, every variable's messages re-read per factor)
-  // only for small runs, where the launch count dominates; past
-  // kFusedMaxStates edge states its two-kernel iteration is faster.
+  // only for small runs, where the launch count dominates; past kFusedMaxBin2
+  // or kFusedMaxStates edge states its two-kernel iteration is faster.
   g->dev.fusable =
       (g->fusable_plan && fuse && (fuse == 2 || chosen || small_run || mode != 2)) ? 1 : 0;
   const bool t0 = (temperature == 0.f);

@@ -90,6 +90,14 @@ constexpr int32_t kMaxBatchPerLaunch = 65535;  // batch elements index grid dime
 constexpr int kTileFactors = 256;
 constexpr int32_t kPairWideTile = -64;  // Tile::pad of tiles run by pair_wide (msets)
 constexpr int32_t kBin2PerThread = 4;  // 2x2 factors per thread in k_fac_phase (msets tiles)
+// Untuned, one launch per iteration (variable sums on the factor side) up to
+// this many edge states per run. 2x2 factors: every thread re-reads the 8
+// messages around its factor, which from about 2^21 edge states on costs more
+// than the second launch (128 x 128 tori, us an iteration: 4 of them 7.5
+// against 10.8, 16 15.3 against 13.8, 96 57.5 against 43.3). Square tables
+// share these sums among more work (64 Potts grids up to 110 x 110 x 8, 7
+// million edge states, 49 against 62; 256 grids, 32 million, 221 against 218).
+constexpr int64_t kFusedMaxBin2 = int64_t(3) << 19;
 constexpr int64_t kFusedMaxStates = int64_t(1) << 24;  // untuned fused shape up to this many
                                                        // edge states per run
 constexpr uint32_t kXcds = 8;  // accelerator complex dies of an MI355X
