@@ -66,17 +66,38 @@ __global__ void k_fill_u32(uint32_t* p, int64_t n, uint32_t v) {
 }
 
 // Normalise and clip incoming messages once at the start of a run
-// (pgmax/infer/bp.py:92-96, :249-259).
+// (pgmax/infer/bp.py:92-96, :249-259), into the engine's layout, in which an
+// edge's states stay together. One thread per edge; the states of an edge of
+// at most kEntryStates are loaded at once and kept for the store (one state
+// after the other, twice, left the loop waiting for each load: 3.1e7 edge
+// states of 2..8 per edge 259 us, now 124).
+constexpr int kEntryStates = 8;
 __global__ void k_normalize_entry(DevGraph g, const float* in, int64_t in_stride, float* out) {
   const int32_t b = blockIdx.y;
   const float* src = in + b * in_stride;
   float* dst = out + b * g.num_es;
   for (int32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < g.num_edges;
        e += gridDim.x * blockDim.x) {
-    const int32_t a = g.edge_es0[e], z = g.edge_es0[e + 1];
+    const int32_t a = g.edge_es0[e], ns = g.edge_es0[e + 1] - a;
+    const int32_t p = g.perm && ns > 0 ? g.perm[a] : a;
     float mx = kNegInf;
-    for (int32_t k = a; k < z; ++k) mx = nmax(mx, src[k]);
-    for (int32_t k = a; k < z; ++k) dst[g.perm ? g.perm[k] : k] = nmax(src[k] - mx, kMsgNegInf);
+    if (ns <= kEntryStates) {
+      float x[kEntryStates];
+#pragma unroll
+      for (int k = 0; k < kEntryStates; ++k)
+        if (k < ns) x[k] = src[a + k];
+#pragma unroll
+      for (int k = 0; k < kEntryStates; ++k)
+        if (k < ns) mx = nmax(mx, x[k]);
+#pragma unroll
+      for (int k = 0; k < kEntryStates; ++k)
+        if (k < ns) dst[p + k] = nmax(x[k] - mx, kMsgNegInf);
+    } else {
+#pragma unroll 4
+      for (int32_t k = 0; k < ns; ++k) mx = nmax(mx, src[a + k]);
+#pragma unroll 4
+      for (int32_t k = 0; k < ns; ++k) dst[p + k] = nmax(src[a + k] - mx, kMsgNegInf);
+    }
   }
 }
 
@@ -775,14 +796,17 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
   }
   // initial messages land in the buffer iteration 0 reads
   float* first = (n_it & 1) ? r.y : r.x;
-  if (d.num_edges > 0) {
+  auto normalise_entry = [&] {
+    if (d.num_edges == 0) return;
     const dim3 grid(std::min<int32_t>((d.num_edges + 255) / 256, 4096), batch);
     hipLaunchKernelGGL(k_normalize_entry, grid, dim3(256), 0, s, d, ftov_in, ftov_in_stride,
                        first);
-  }
+  };
   PGX_HIP(hipGetLastError());
   if (d.num_tasks == 0 || d.num_es == 0) {
     // no factors: every iteration maps the (empty) messages onto themselves
+    normalise_entry();
+    PGX_HIP(hipGetLastError());
     if (first != r.x && d.num_es > 0)
       PGX_HIP(hipMemcpyAsync(r.x, first, msg_bytes, hipMemcpyDeviceToDevice, s));
     return PGX_OK;
@@ -868,12 +892,6 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
   g->dev.fusable =
       (g->fusable_plan && fuse && (fuse == 2 || chosen || small_run || mode != 2)) ? 1 : 0;
   const bool t0 = (temperature == 0.f);
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
-  if (prof) {
-    PGX_HIP(hipEventCreate(&ev0));
-    PGX_HIP(hipEventCreate(&ev1));
-    PGX_HIP(hipEventRecord(ev0, s));
-  }
   KernelClock clk;
   clk.on = prof == 2;
   clk.s = s;
@@ -884,15 +902,29 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
     if (mode == 1) mode = 2;
   }
   // graphs of 2x2 factors and variables of <= 4 edges: the per-phase shape
-  // iterates on one float per message. The entry normalisation wrote full
-  // pairs into `first`; pack them into the other buffer and swap the
-  // buffers' roles, so iteration 0 reads the packed copy and the last
-  // iteration writes r.x (unpacked into ftov_out below).
+  // iterates on one float per message. They enter packed, into the other
+  // buffer, and the buffers swap roles, so iteration 0 reads the packed
+  // messages and the last iteration writes r.x (unpacked into ftov_out below).
   g->dev.packed = (mode == 2 && !g->dev.bip && g->packed_plan && g->dev.even2 && pack) ? 1 : 0;
   if (g->dev.packed) {
-    float* other = (first == r.x) ? r.y : r.x;
-    launch_pair_pack(g->dev, first, other, d.num_es, batch, s);
     std::swap(r.x, r.y);
+    launch_pair_entry(g->dev, ftov_in, ftov_in_stride, nullptr, (n_it & 1) ? r.y : r.x, d.num_es,
+                      batch, s);
+  } else if (mode == 2 && g->dev.bip) {
+    // pairs for the chunk sums of the initial messages, one float per message
+    // for the iterations
+    float *full, *m0, *m1;
+    bip_buffers(g->dev, r, batch, &full, &m0, &m1);
+    launch_pair_entry(g->dev, ftov_in, ftov_in_stride, full, m0, d.num_es / 2, batch, s);
+  } else {
+    normalise_entry();
+  }
+  PGX_HIP(hipGetLastError());
+  hipEvent_t ev0 = nullptr, ev1 = nullptr;
+  if (prof) {
+    PGX_HIP(hipEventCreate(&ev0));
+    PGX_HIP(hipEventCreate(&ev1));
+    PGX_HIP(hipEventRecord(ev0, s));
   }
   if (mode == 1)
     clk.run(PGX_KERNEL_TASK_LOOP, [&] {

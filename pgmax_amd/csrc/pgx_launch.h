@@ -340,9 +340,10 @@ void launch_converge_finish(pgx_graph* g, const RunBufs& r, float* out, int32_t 
                             hipStream_t s);
 template <bool kT0>
 int launch_coop(pgx_graph* g, const RunBufs& r, int32_t batch, hipStream_t s, int64_t tile);
-// one float per binary message: engine-layout pairs -> packed, packed -> caller layout
-void launch_pair_pack(const DevGraph& d, const float* full, float* packed, int64_t stride,
-                      int32_t batch, hipStream_t s);
+// one float per binary message: caller's messages -> normalised and packed (and
+// engine-layout pairs in full, if not null), packed -> caller's layout
+void launch_pair_entry(const DevGraph& d, const float* in, int64_t in_stride, float* full,
+                       float* packed, int64_t stride, int32_t batch, hipStream_t s);
 void launch_pair_unpack(const DevGraph& d, const float* packed, int64_t stride, float* out,
                         int32_t batch, hipStream_t s);
 // the plugin API: one block kind's update on given vtof, for `batch` elements

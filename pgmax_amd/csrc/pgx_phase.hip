@@ -1,7 +1,7 @@
 // Per-phase shape: every BP iteration is a few launches over the whole
 // (batched) graph -- the variable phase, then one factor-phase launch per
 // block kind -- or one launch for graphs whose factor side recomputes
-// variable sums. Also the one-float message pack / unpack passes and the
+// variable sums. Also the one-float message entry and unpack passes and the
 // plugin API's one-type factor update.
 
 #include <hip/hip_cooperative_groups.h>
@@ -16,30 +16,44 @@ namespace {
 
 // Complete bipartite graphs, and in the per-phase shape all graphs of 2x2
 // factors whose variables have at most 4 edges, iterate on one float per
-// binary edge (pair_encode), stride floats per batch element. k_pair_pack
-// turns the engine-layout messages (planar pairs) into that form;
-// k_pair_unpack writes the caller's reference layout from it.
-__global__ void k_pair_pack(DevGraph g, const float* full, float* packed, int64_t stride) {
+// binary edge (pair_encode), stride floats per batch element. k_pair_entry
+// normalises and clips the caller's messages (pgmax/infer/bp.py:92-96) and
+// writes them in that form, and as engine-layout pairs where a run needs both
+// (full not null); k_pair_unpack writes the caller's layout from it. One
+// thread per edge, both states in one access (3.2 million edges of 64 RBMs:
+// normalising to pairs, packing those and unpacking by single states took
+// 31 + 14 + 31 us, the two kernels take 20 + 19). Every edge has two states,
+// which stay together in the engine's layout at an even offset.
+template <bool kFull>
+__global__ void __launch_bounds__(256)
+    k_pair_entry(DevGraph g, const float* in, int64_t in_stride, float* full, float* packed,
+                 int64_t stride) {
   const int32_t b = blockIdx.y;
-  const int64_t npair = g.num_es / 2;
-  const float* src = full + b * g.num_es;
+  const float* src = in + b * in_stride;
   float* dst = packed + b * stride;
-  for (int64_t i = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; i < npair;
-       i += int64_t(gridDim.x) * blockDim.x) {
-    const float2 m = ld2(src + 2 * i);
-    dst[i] = pair_encode(m.x, m.y);
+  for (int64_t e = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; e < g.num_edges;
+       e += int64_t(gridDim.x) * blockDim.x) {
+    float x[2];
+    ldv<2>(src + 2 * e, x);
+    const int32_t p = g.perm[2 * e];
+    const float mx = nmax(x[0], x[1]);
+    x[0] = nmax(x[0] - mx, kMsgNegInf);
+    x[1] = nmax(x[1] - mx, kMsgNegInf);
+    if (kFull) stv<2>(full + b * g.num_es + p, x);
+    dst[p >> 1] = pair_encode(x[0], x[1]);
   }
 }
 
-__global__ void k_pair_unpack(DevGraph g, const float* packed, int64_t stride, float* out) {
+__global__ void __launch_bounds__(256)
+    k_pair_unpack(DevGraph g, const float* packed, int64_t stride, float* out) {
   const int32_t b = blockIdx.y;
   const float* src = packed + b * stride;
   float* dst = out + b * g.num_es;
-  for (int64_t k = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; k < g.num_es;
-       k += int64_t(gridDim.x) * blockDim.x) {
-    const int32_t p = g.perm[k];
-    const float2 m = pair_decode(src[p >> 1]);
-    dst[k] = (p & 1) ? m.y : m.x;
+  for (int64_t e = blockIdx.x * int64_t(blockDim.x) + threadIdx.x; e < g.num_edges;
+       e += int64_t(gridDim.x) * blockDim.x) {
+    const float2 m = pair_decode(src[g.perm[2 * e] >> 1]);
+    const float x[2] = {m.x, m.y};
+    stv<2>(dst + 2 * e, x);
   }
 }
 
@@ -501,17 +515,23 @@ void launch_var_phase(const DevGraph& d, const float* m, int64_t m_stride, const
     });
 }
 
-void launch_pair_pack(const DevGraph& d, const float* full, float* packed, int64_t stride,
-                      int32_t batch, hipStream_t s) {
-  hipLaunchKernelGGL(k_pair_pack,
-                     dim3(unsigned(std::min<int64_t>((d.num_es / 2 + 255) / 256, 2048)), batch),
-                     dim3(256), 0, s, d, full, packed, stride);
+static dim3 edge_grid(const DevGraph& d, int32_t batch) {
+  return dim3(unsigned(std::min<int64_t>((int64_t(d.num_edges) + 255) / 256, 2048)), batch);
+}
+
+void launch_pair_entry(const DevGraph& d, const float* in, int64_t in_stride, float* full,
+                       float* packed, int64_t stride, int32_t batch, hipStream_t s) {
+  if (full)
+    hipLaunchKernelGGL((k_pair_entry<true>), edge_grid(d, batch), dim3(256), 0, s, d, in,
+                       in_stride, full, packed, stride);
+  else
+    hipLaunchKernelGGL((k_pair_entry<false>), edge_grid(d, batch), dim3(256), 0, s, d, in,
+                       in_stride, full, packed, stride);
 }
 
 void launch_pair_unpack(const DevGraph& d, const float* packed, int64_t stride, float* out,
                         int32_t batch, hipStream_t s) {
-  const dim3 ugrid(unsigned(std::min<int64_t>((d.num_es + 255) / 256, 2048)), batch);
-  hipLaunchKernelGGL(k_pair_unpack, ugrid, dim3(256), 0, s, d, packed, stride, out);
+  hipLaunchKernelGGL(k_pair_unpack, edge_grid(d, batch), dim3(256), 0, s, d, packed, stride, out);
 }
 
 template <bool kT0, bool kConv>
@@ -573,14 +593,12 @@ static int launch_phased_t(pgx_graph* g, const RunBufs& r, int32_t batch, hipStr
   const TileSet& T = g->tsets[tile <= 64 ? 0 : (tile <= 128 ? 1 : 2)];
   const dim3 fgrid(T.num_tiles, batch);
   if (d.bip) {
-    // chunk sums of the initial messages, their one-float form, then one
-    // launch per iteration alternating between two message buffers and two
-    // chunk-sum buffers (run_impl unpacks the last message buffer)
+    // chunk sums of the initial messages, then one launch per iteration
+    // alternating between two message buffers and two chunk-sum buffers
+    // (run_impl writes the first message buffer and unpacks the last)
     float *first, *m0, *m1;
     bip_buffers(d, r, batch, &first, &m0, &m1);
     launch_var_phase(d, first, d.num_es, r.ev, r.ev_stride, r.vsum, r.partial, batch, s, &clk);
-    hipLaunchKernelGGL(k_pair_pack, dim3(unsigned(std::min<int64_t>((d.num_es / 2 + 255) / 256, 2048)), batch),
-                       dim3(256), 0, s, d, first, m0, d.num_es / 2);
     float* p0 = r.partial;
     float* p1 = r.partial + size_t(batch) * size_t(d.partial_size);
     clk.run_n(PGX_KERNEL_BIPARTITE, r.n_it, [&] {

@@ -139,3 +139,49 @@ def test_short_lane_tiles_match_oracle(gpu, tile, temperature):
     np.testing.assert_array_equal(_np(out), ref)
     np.testing.assert_array_equal(_np(d), ref_d)
   bb.close()
+
+
+@pytest.mark.parametrize("kind", ["torus", "bipartite", "unary", "mixed"])
+@pytest.mark.parametrize("offset", [0, 1, 3])
+@pytest.mark.parametrize("iters", [1, 2])
+def test_entry_messages_at_any_alignment(gpu, kind, offset, iters):
+  """Messages enter normalised and clipped in each engine layout, from buffers
+  at any float alignment, with non-finite states."""
+  import torch
+  from pgmax_amd import batch
+  from pgmax_amd import engine
+  if kind == "torus":
+    w = batch.grid_wiring(5, 7, 2, torus=True, full_tables=True)
+  elif kind == "mixed":  # 2, 3, 9 and 12 states
+    w = batch.BatchedBP([batch.grid_wiring(3, 3, s, full_tables=True) for s in (2, 3, 9, 12)],
+                        temperature=1.0).union
+  else:
+    h, v = vgroup.NDVarArray(num_states=2, shape=(33,)), vgroup.NDVarArray(num_states=2, shape=(35,))
+    fg = fgraph.FactorGraph(variable_groups=[h, v])
+    if kind == "unary":
+      for g, n in ((h, 33), (v, 35)):
+        fg.add_factors(fgroup.EnumFactorGroup(variables_for_factors=[[g[i]] for i in range(n)],
+                                              factor_configs=np.arange(2)[:, None]))
+    fg.add_factors(fgroup.PairwiseFactorGroup(
+        variables_for_factors=[[h[i], v[j]] for i in range(33) for j in range(35)]))
+    w = None
+    eng = infer.BP(fg.bp_state, temperature=1.0).context
+    graph = lbp.graph_from_context(eng)
+    eng = eng.engine
+  if w is not None:
+    eng, graph = engine.Engine.from_wiring(w.to_engine_wiring()), lbp.graph_from_flat(w)
+  g, rng = eng.graph, np.random.default_rng(11)
+  ft = rng.normal(0, 3, size=(3, g.num_es)).astype(np.float32)
+  ft[0, ::7] = -3e38
+  ft[1, 1::11] = -np.inf
+  ft[2, 2::13] = np.inf
+  ft[2, 5::17] = np.nan
+  lp = rng.normal(size=(3, g.num_lp)).astype(np.float32)
+  ev = rng.normal(size=g.num_vs).astype(np.float32)
+  buf = torch.zeros(ft.size + offset, device="cuda")
+  buf[offset:] = torch.as_tensor(ft.reshape(-1), device="cuda")
+  out, d = eng.run(lp, buf[offset:].view(3, -1), ev, iters, 0.5, 1.0)
+  for b in range(3):
+    ref, ref_d = lbp.run_with_diffs(graph, lp[b], ft[b], ev, iters, 0.5, 1.0)
+    np.testing.assert_array_equal(_np(out)[b], ref)
+    np.testing.assert_array_equal(_np(d)[b], ref_d)
