@@ -279,14 +279,16 @@ int pgx_enum_rows_fac_to_var(const int32_t* cfg_row_ptr, const int32_t* row_es,
 
 /* Engine options: "mode" (0 auto, 1 one workgroup per task, 2 per-phase
  * launches, 3 one cooperative launch for all iterations of a graph whose
- * factor side recomputes variable sums, see "fuse"), "block" (threads per
+ * factor side recomputes variable sums, see "fuse", 4 patches: small graphs of
+ * 2x2 factors, several iterations per launch), "block" (threads per
  * workgroup of the task loop and of the complete bipartite iteration:
  * 128, 256 or 512 there; 0 auto), "profile" (1: record
  * HIP events around the BP iterations of every pgx_run; 2: also around every
  * kernel launch), "fuse" (1, the
  * default: graphs of pairwise factors whose variables have at most 8 edges
  * recompute variable sums on the factor side -- without tuning only for
- * runs of at most 2^24 edge states; 2: at every size --, and complete
+ * runs of at most 2^24 edge states, 1.5 * 2^20 with 2x2 tables only; 2: at
+ * every size --, and complete
  * bipartite binary graphs (a binary RBM) form them from chunk sums the factor
  * kernel leaves behind -- one launch per iteration either way; 0: separate
  * variable phase),

@@ -1,14 +1,16 @@
 // Kernels and C ABI of the loopy-BP engine (include/pgx.h).
 //
-// Two execution shapes for pgx_run, chosen per call:
+// Execution shapes for pgx_run, chosen per call:
 //   * task loop: one workgroup owns one independent component of one batch
 //     element and runs every iteration of it in a single launch; variable
 //     and factor phases are separated by workgroup barriers only, so the
 //     graph's working set stays in that CU's caches.
+//   * patches (pgx_patch.hip): small graphs of 2x2 factors, several
+//     iterations per launch on overlapping patches in LDS.
 //   * phased: per iteration one launch for the variable phase and one for
 //     the factor phase over the whole (batched) graph; used when there are
 //     too few independent components to fill the GPU.
-// Both run the same per-factor device code (pgx_device.h).
+// All run the same per-factor arithmetic (pgx_device.h).
 
 #include <hip/hip_cooperative_groups.h>
 #include <hip/hip_runtime.h>
@@ -439,6 +441,19 @@ int pgx_graph_create(const pgx_wiring* wiring, pgx_graph** out) {
     for (int k = 0; k < 8; ++k) d.bip_aff[k] = P.bip_aff[k];
     g->bip_plan = 1;
   }
+  {
+    const Patches ps = build_patches(P);
+    if (ps.count > 0) {
+      int32_t *desc, *thr, *lpo, *extra;
+      if ((rc = up(ps.desc, &desc)) || (rc = up(ps.thr, &thr)) || (rc = up(ps.lp, &lpo)) ||
+          (rc = up(ps.extra, &extra))) {
+        pgx_graph_destroy(g);
+        return rc;
+      }
+      g->patches = DevPatches{ps.count, ps.depth, ps.threads, reinterpret_cast<const int4*>(desc),
+                              reinterpret_cast<const int4*>(thr), lpo, extra};
+    }
+  }
   d.fusable = (P.pairwise_only && P.max_degree <= kFuseMaxDeg) ? 1 : 0;
   g->packed_plan = P.packable ? 1 : 0;
   g->even2_plan = P.even2;
@@ -655,6 +670,19 @@ static std::pair<int64_t, int64_t> converge_shape(const pgx_graph* g, int32_t ba
   if (bin2 && factors >= 512) return {1, wgs <= 512 ? 1024 : 512};
   if ((g->kinds_mask & ~kKindsPairwise) == 0 && factors >= 256) return {1, 512};
   return {1, 256};
+}
+
+// Untuned runs take k_patch where the graph is small enough: whole components
+// always (16 x 16 tori, us an iteration at T = 1 against the task loop's 512
+// threads: one 1.5 and 3.9, 256 of them 1.7 and 4.1, 1,000 6.1 and 8.2),
+// patches with rings while the repeated factors run on idle CUs (against one
+// launch an iteration, T = 1: 50 x 50 torus 1.9 and 5.9, 16 of them 4.2 and 6.7,
+// 128 x 128 3.7 and 6.3, two 6.3 and 6.5, four 10.9 and 7.3; T = 0: 100 of
+// 24 x 24 4.3 and 6.4, four of 128 x 128 7.5 and 6.8).
+static bool patches_pay(const pgx_graph* g, int32_t batch, bool t0) {
+  if (g->patches.count == 0) return false;
+  const int64_t most = t0 ? int64_t(3) << 15 : int64_t(1) << 16;  // factors
+  return g->patches.depth == 0 || int64_t(g->plan.num_factors) * batch <= most;
 }
 
 // Delta slots per (batch element, iteration) of the per-launch kernels:
@@ -875,7 +903,9 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
     mode = shape.first;
     if (bs == 0) bs = shape.second;
   }
-  if (converge && mode == 3) mode = 1;
+  if (converge && mode >= 3) mode = 1;
+  if (mode == 0 && fuse && pack && patches_pay(g, batch, temperature == 0.f)) mode = 4;
+  if (mode == 4 && g->patches.count == 0) mode = 2;
   if (mode == 0) {
     // One workgroup per task pays when there are enough tasks to fill the
     // CUs and each is small enough that a CU's sweep over it is shorter than
@@ -916,7 +946,7 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
     float *full, *m0, *m1;
     bip_buffers(g->dev, r, batch, &full, &m0, &m1);
     launch_pair_entry(g->dev, ftov_in, ftov_in_stride, full, m0, d.num_es / 2, batch, s);
-  } else {
+  } else if (mode != 4) {  // (k_patch reads the caller's messages itself)
     normalise_entry();
   }
   PGX_HIP(hipGetLastError());
@@ -935,23 +965,28 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
     clk.run(PGX_KERNEL_FAC_FUSED, [&] {
       rc = t0 ? launch_coop<true>(g, r, batch, s, tile) : launch_coop<false>(g, r, batch, s, tile);
     });
+  else if (mode == 4)
+    clk.run(PGX_KERNEL_FAC_FUSED, [&] {
+      rc = launch_patches(g, r, ftov_in, ftov_in_stride, ftov_out, scr, batch, t0, s);
+    });
   else {
     // reading shared tables pays when the one pass that finds them is short
     // next to the run (it reads every table once)
     if (!(share && n_it >= 8)) r.share_mem = nullptr;
     rc = t0 ? launch_phased<true>(g, r, batch, s, clk, tile, bs, lanes != 0, lset)
             : launch_phased<false>(g, r, batch, s, clk, tile, bs, lanes != 0, lset);
-    if (rc == PGX_OK && r.dslot_n > 1) {  // the per-launch kernels wrote delta slots
-      const int64_t nd = int64_t(batch) * n_it;
-      hipLaunchKernelGGL(k_delta_reduce, dim3(std::min<int64_t>((nd + 255) / 256, 1024)),
-                         dim3(256), 0, s, r.dslot, r.dslot_n, r.deltas, nd);
-      PGX_HIP(hipGetLastError());
-    }
+  }
+  if (rc == PGX_OK && mode != 1 && mode != 3 && r.dslot_n > 1) {
+    // the per-launch kernels wrote delta slots
+    const int64_t nd = int64_t(batch) * n_it;
+    hipLaunchKernelGGL(k_delta_reduce, dim3(std::min<int64_t>((nd + 255) / 256, 1024)), dim3(256),
+                       0, s, r.dslot, r.dslot_n, r.deltas, nd);
+    PGX_HIP(hipGetLastError());
   }
   if (rc == PGX_OK && converge && mode == 2) {
     launch_converge_finish(g, r, ftov_out, batch, s);
     PGX_HIP(hipGetLastError());
-  } else if (rc == PGX_OK && planar) {
+  } else if (rc == PGX_OK && planar && mode != 4) {
     const dim3 ugrid(unsigned(std::min<int64_t>((d.num_es + 255) / 256, 2048)), batch);
     if (mode == 2 && g->dev.bip) {  // the last one-float message buffer
       float *full, *m0, *m1;
@@ -1192,6 +1227,7 @@ int pgx_autotune(pgx_graph* g, const float* lp, int64_t lp_stride, const float* 
   if (converge)  // per-phase launches that skip the tasks that are done
     for (int fi = g->fusable_plan ? 0 : 1; fi < 2; ++fi)
       for (int64_t t : {64, 128, 256}) cands.push_back(RunCfg{2, 0, fi == 0 ? 1 : 0, 3, t});
+  if (!converge && g->patches.count > 0) cands.push_back(RunCfg{4, 0, 1, 3, 256});
   if (!converge && g->fusable_plan)
     for (int64_t t : {64, 256}) cands.push_back(RunCfg{3, 0, 1, 3, t});
   // the task loop last, so its probes can stop early against the best shape

@@ -253,6 +253,15 @@ struct Tile {
   int32_t block, i0, i1, pad;
 };
 
+// Plan's Patches on the device.
+struct DevPatches {
+  int32_t count = 0, depth = 0, threads = 0;
+  const int4* desc = nullptr;
+  const int4* thr = nullptr;
+  const int32_t* lp = nullptr;
+  const int32_t* extra = nullptr;
+};
+
 // Execution shape of one run: mode 1 task loop / 2 phased, workgroup size of
 // the task loop, factor-side variable sums, vector accesses.
 struct RunCfg {
@@ -314,6 +323,7 @@ struct pgx_graph {
   int32_t num_tiles = 0;
   int32_t fusable_plan = 0;
   int32_t bip_plan = 0;     // complete bipartite binary graph (k_bipartite applies)
+  pgx::DevPatches patches;  // count 0: none
   int32_t packed_plan = 0;  // 2x2 factors only, binary variables of <= 4 edges (Plan::packable)
   bool even2_plan = false;  // 2-state edges / variables at even offsets
   int32_t* zero_strides = nullptr;  // NHC zeros: chunk strides of the reference layout
@@ -340,6 +350,11 @@ void launch_converge_finish(pgx_graph* g, const RunBufs& r, float* out, int32_t 
                             hipStream_t s);
 template <bool kT0>
 int launch_coop(pgx_graph* g, const RunBufs& r, int32_t batch, hipStream_t s, int64_t tile);
+// pgx_patch.hip: a run in launches of patches.depth iterations (0: one launch),
+// from the caller's messages to the caller's result; buf holds two floats per
+// edge and batch element
+int launch_patches(pgx_graph* g, const RunBufs& r, const float* ftov_in, int64_t in_stride,
+                   float* out, float* buf, int32_t batch, bool t0, hipStream_t s);
 // one float per binary message: caller's messages -> normalised and packed (and
 // engine-layout pairs in full, if not null), packed -> caller's layout
 void launch_pair_entry(const DevGraph& d, const float* in, int64_t in_stride, float* full,

@@ -763,4 +763,142 @@ int build_plan(const pgx_wiring& w, Plan* P, std::string* err, int64_t merge_bel
   return PGX_OK;
 }
 
+namespace {
+
+// Factors of a graph of 2x2 factors as nodes, joined by shared variables.
+struct FactorNeighbours {
+  const Plan& P;
+  template <class F>
+  void each(int32_t f, F&& fn) const {
+    for (int32_t e = 2 * f; e < 2 * f + 2; ++e) {
+      const int32_t v = P.edge_var[e];
+      for (int32_t p = P.var_eptr[v]; p < P.var_eptr[v + 1]; ++p) {
+        const int32_t o = P.var_adj_es_ref[p] / 4;  // edge state -> factor
+        if (o != f) fn(o);
+      }
+    }
+  }
+};
+
+// Splits `fs` into pieces of at most `own` factors, each compact: halves of
+// the breadth-first order from a factor at the far end, recursively.
+void split_compact(const FactorNeighbours& nb, std::vector<int32_t> fs, int32_t own,
+                   std::vector<int32_t>* mark, int32_t* stamp,
+                   std::vector<std::vector<int32_t>>* out) {
+  if (int32_t(fs.size()) <= own) {
+    out->push_back(std::move(fs));
+    return;
+  }
+  const int32_t in = ++*stamp;
+  for (int32_t f : fs) (*mark)[f] = in;
+  std::vector<int32_t> order;
+  auto sweep = [&](int32_t start, int32_t from, int32_t to) {
+    order.clear();
+    size_t next = 0;
+    auto visit = [&](int32_t f) {
+      if ((*mark)[f] == from) {
+        (*mark)[f] = to;
+        order.push_back(f);
+      }
+    };
+    visit(start);
+    for (size_t h = 0; order.size() < fs.size(); ++h) {
+      while (h == order.size()) visit(fs[next++]);  // another component
+      nb.each(order[h], visit);
+    }
+  };
+  sweep(fs[0], in, in + 1);
+  const int32_t far = order.back();
+  sweep(far, in + 1, in + 2);
+  *stamp = in + 2;
+  const int32_t pieces = (int32_t(fs.size()) + own - 1) / own;
+  const size_t cut = size_t(int64_t(fs.size()) * (pieces / 2) / pieces);
+  split_compact(nb, std::vector<int32_t>(order.begin(), order.begin() + cut), own, mark, stamp,
+                out);
+  split_compact(nb, std::vector<int32_t>(order.begin() + cut, order.end()), own, mark, stamp, out);
+}
+
+}  // namespace
+
+Patches build_patches(const Plan& P) {
+  const int32_t F = P.num_factors;
+  if (F == 0 || P.max_degree > 4 || P.num_edges != 2 * F) return {};
+  std::vector<int32_t> lp0(static_cast<size_t>(F));
+  int32_t largest = 0;  // factors of a task
+  for (const Task& t : P.tasks) {
+    int32_t n = 0;
+    for (int32_t bi = t.b0; bi < t.b1; ++bi) {
+      const Block& b = P.blocks[bi];
+      if (b.kind != kEnumBin2) return {};
+      n += b.count;
+      for (int32_t i = 0; i < b.count; ++i) lp0[b.f0 + i] = int32_t(b.c0 + 4 * i);
+    }
+    largest = std::max(largest, n);
+  }
+  const FactorNeighbours nb{P};
+  std::vector<std::vector<int32_t>> owns;
+  Patches out;
+  if (2 * largest <= kPatchThreads) {
+    for (const Task& t : P.tasks) {
+      owns.emplace_back();
+      for (int32_t bi = t.b0; bi < t.b1; ++bi)
+        for (int32_t i = 0; i < P.blocks[bi].count; ++i) owns.back().push_back(P.blocks[bi].f0 + i);
+    }
+  } else if (F <= kPatchMaxFactors) {
+    out.depth = kPatchDepth;
+    std::vector<int32_t> all(static_cast<size_t>(F)), mark(static_cast<size_t>(F), 0);
+    std::iota(all.begin(), all.end(), 0);
+    int32_t stamp = 0;
+    split_compact(nb, std::move(all), kPatchOwn, &mark, &stamp, &owns);
+  } else {
+    return {};
+  }
+  // local[f]: position of factor f in the patch being built, or -1
+  std::vector<int32_t> local(static_cast<size_t>(F), -1), slot(static_cast<size_t>(2 * F), -1);
+  for (std::vector<int32_t>& fs : owns) {
+    const int32_t own = int32_t(fs.size());
+    std::vector<int32_t> ring(fs.size(), 0);
+    for (int32_t i = 0; i < own; ++i) local[fs[i]] = i;
+    for (int32_t h = 0; h < int32_t(fs.size()); ++h)  // (fs grows ring by ring)
+      if (ring[h] + 1 < out.depth)
+        nb.each(fs[h], [&](int32_t f) {
+          if (local[f] >= 0) return;
+          local[f] = int32_t(fs.size());
+          fs.push_back(f);
+          ring.push_back(ring[h] + 1);
+        });
+    const int32_t nt = 2 * int32_t(fs.size());
+    if (nt > kPatchThreads) return {};
+    const int32_t t0 = int32_t(out.lp.size()), x0 = int32_t(out.extra.size());
+    for (int32_t t = 0; t < nt; ++t) {
+      const int32_t f = fs[t / 2], e = 2 * f + t % 2, v = P.edge_var[e];
+      uint32_t s[4] = {0xffffu, 0xffffu, 0xffffu, 0xffffu};
+      for (int32_t p = P.var_eptr[v], k = 0; p < P.var_eptr[v + 1]; ++p, ++k) {
+        const int32_t o = P.var_adj_es_ref[p] / 2;
+        if (local[o / 2] >= 0) {
+          s[k] = uint32_t(2 * local[o / 2] + o % 2);
+        } else {
+          if (slot[o] < 0) {
+            slot[o] = nt + int32_t(out.extra.size()) - x0;
+            out.extra.push_back(o);
+          }
+          s[k] = uint32_t(slot[o]);
+        }
+      }
+      out.thr.insert(out.thr.end(),
+                     {int32_t(uint32_t(e) | uint32_t(ring[t / 2]) << kPatchRingShift),
+                      P.edge_vs0[e], int32_t(s[0] | s[1] << 16), int32_t(s[2] | s[3] << 16)});
+      out.lp.push_back(lp0[f]);
+    }
+    const int32_t nx = int32_t(out.extra.size()) - x0;
+    if (nt + nx > kPatchSlots) return {};
+    out.desc.insert(out.desc.end(), {t0, nt, x0, nx, 2 * own, 0, 0, 0});
+    out.threads = std::max(out.threads, (nt + 63) / 64 * 64);
+    for (int32_t f : fs) local[f] = -1;
+    for (int32_t k = x0; k < x0 + nx; ++k) slot[out.extra[k]] = -1;
+  }
+  out.count = int32_t(owns.size());
+  return out;
+}
+
 }  // namespace pgx

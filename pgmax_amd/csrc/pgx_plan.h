@@ -172,6 +172,33 @@ struct Plan {
   int32_t bip_aff[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 };
 
+// Patches of a small graph of 2x2 factors whose variables have at most 4
+// edges (k_patch): each workgroup's own factors and the rings around them.
+// depth 0: every patch is whole components and needs no rings; else a patch
+// holds the factors within depth - 1 steps of its own, and the edges one step
+// further out are only read (extra). One thread per edge, a factor's two
+// edges side by side, own factors first, then ring by ring.
+struct Patches {
+  int32_t count = 0, depth = 0;
+  int32_t threads = 0;            // most threads of a patch
+  std::vector<int32_t> desc;      // 8 per patch: [first thread, threads, first extra,
+                                  // extras, own threads, 0, 0, 0]
+  std::vector<int32_t> thr;       // 4 per thread: [edge | ring << kPatchRingShift, first
+                                  // variable state, LDS slots of its variable's edges in
+                                  // edge order, 16 bits each (0xffff: none)]
+  std::vector<int32_t> lp;        // per thread: first log-potential of its factor
+  std::vector<int32_t> extra;     // edges
+};
+constexpr int32_t kPatchThreads = 1024;
+constexpr int32_t kPatchSlots = 2048;        // LDS message slots: threads, then extras
+constexpr int32_t kPatchDepth = 4;
+constexpr int32_t kPatchOwn = 80;            // own factors aimed at with rings
+constexpr int32_t kPatchMaxFactors = 1 << 15;  // of a graph with rings
+constexpr int32_t kPatchRingShift = 28;
+constexpr int32_t kPatchEdgeMask = (1 << kPatchRingShift) - 1;
+// Empty when the graph is of another kind or too large.
+Patches build_patches(const Plan& plan);
+
 // Builds `plan` from the wiring. Neighbouring components whose combined
 // edge + variable states stay below merge_below share one task (0: never).
 // Returns PGX_OK or an error code with `err`.

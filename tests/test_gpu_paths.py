@@ -185,3 +185,60 @@ def test_entry_messages_at_any_alignment(gpu, kind, offset, iters):
     ref, ref_d = lbp.run_with_diffs(graph, lp[b], ft[b], ev, iters, 0.5, 1.0)
     np.testing.assert_array_equal(_np(out)[b], ref)
     np.testing.assert_array_equal(_np(d)[b], ref_d)
+
+
+def _binary_graph(kind):
+  from pgmax_amd import batch
+  grid = lambda h, w, torus: batch.grid_wiring(h, w, 2, torus=torus, full_tables=True)
+  if kind == "tiny":
+    return grid(1, 2, False)
+  if kind == "whole":  # 512 factors: a workgroup's last
+    return grid(16, 16, True)
+  if kind == "rings":  # 544: the first with rings
+    return grid(17, 16, True)
+  if kind == "open":
+    return grid(41, 30, False)
+  if kind == "chain":
+    return grid(1, 801, False)
+  if kind == "union":  # components of a workgroup each, merged and not
+    return batch.BatchedBP([grid(n, n, True) for n in (3, 9, 3, 16, 12)], temperature=1.0).union
+  if kind == "parallel":  # two factors on every other pair
+    pairs = [[i, i + 1] for i in range(799)] + [[i, i + 1] for i in range(0, 799, 2)]
+    return batch.pairwise_wiring(800, 2, np.array(pairs), full_tables=True)
+  rng = np.random.default_rng(0)  # rings grow past a workgroup: no patches
+  pairs = np.concatenate([np.sort(rng.permutation(900).reshape(-1, 2), 1) for _ in range(3)])
+  return batch.pairwise_wiring(900, 2, np.unique(pairs, axis=0), full_tables=True)
+
+
+@pytest.mark.parametrize("kind", ["tiny", "whole", "rings", "open", "chain", "union", "parallel",
+                                  "random"])
+@pytest.mark.parametrize("temperature", [0.0, 0.35, 1.0])
+@pytest.mark.parametrize("iters", [1, 4, 7])
+def test_patches_match_oracle(gpu, kind, temperature, iters):
+  """Several iterations per launch on patches: the oracle's messages and
+  deltas, with fewer, exactly and more iterations than rings, batched, from
+  buffers at an odd float offset, with non-finite tables and evidence."""
+  import torch
+  from pgmax_amd import engine
+  w = _binary_graph(kind)
+  eng, graph = engine.Engine.from_wiring(w.to_engine_wiring()), lbp.graph_from_flat(w)
+  g, rng = eng.graph, np.random.default_rng(13)
+  def shifted(x):
+    buf = torch.zeros(x.size + 1, device="cuda")
+    buf[1:] = torch.as_tensor(x.reshape(-1), device="cuda")
+    return buf[1:].view(x.shape)
+  ft = rng.normal(size=(2, g.num_es)).astype(np.float32)
+  lp = rng.normal(size=(2, g.num_lp)).astype(np.float32)
+  ev = rng.normal(size=(2, g.num_vs)).astype(np.float32)
+  lp[1, 1] = np.inf
+  lp[1, -1] = np.nan
+  ev[1, g.num_vs // 2] = -np.inf
+  _lib.set_option("mode", 4)
+  out, d = eng.run(shifted(lp), shifted(ft), shifted(ev), iters, 0.5, temperature)
+  _lib.set_option("mode", 0)
+  auto, auto_d = eng.run(lp, ft, ev, iters, 0.5, temperature)
+  for b in range(2):
+    ref, ref_d = lbp.run_with_diffs(graph, lp[b], ft[b], ev[b], iters, 0.5, temperature)
+    for o, od in ((out, d), (auto, auto_d)):
+      np.testing.assert_array_equal(_np(o)[b], ref)
+      np.testing.assert_array_equal(_np(od)[b], ref_d)
