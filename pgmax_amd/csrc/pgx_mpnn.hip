@@ -53,7 +53,7 @@ static_assert(kNumParams == PGX_MPNN_NUM_PARAMS, "parameter layout");
 constexpr int kLayerPart = kKZ * kH + kH;  // per-workgroup partial of dW_l, db_l
 constexpr int kEmbedPart = kNin * kH + kH;
 constexpr int kHeadPart = kH + 1;
-constexpr int kMaxLayerBlocks = 1024;
+constexpr int kMaxLayerBlocks = 512;  // workgroups of k_mp_layer_wgrad: two per CU
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -80,8 +80,6 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
 }
 __device__ __forceinline__ float bf2f(u16 h) { return __uint_as_float(uint32_t(h) << 16); }
-__device__ __forceinline__ float ld(const u16* p) { return bf2f(*p); }
-__device__ __forceinline__ float ld(const float* p) { return *p; }
 
 // D += A B for a 16x32 A and 32x16 B in BF16. Lane l holds A[l % 16][8(l/16) .. +7],
 // B[8(l/16) .. +7][l % 16] and D[4(l/16) .. +3][l % 16].
@@ -180,15 +178,6 @@ __device__ __forceinline__ void load8(const u16* p, float* x) {
   for (int k = 0; k < 4; ++k) {
     x[2 * k] = bf2f(u16(v[k] & 0xffffu));
     x[2 * k + 1] = bf2f(u16(v[k] >> 16));
-  }
-}
-__device__ __forceinline__ void load8(const float* p, float* x) {
-  const f32x4 a = *reinterpret_cast<const f32x4*>(p);
-  const f32x4 c = *reinterpret_cast<const f32x4*>(p + 4);
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    x[k] = a[k];
-    x[4 + k] = c[k];
   }
 }
 
@@ -298,16 +287,15 @@ __global__ void __launch_bounds__(kThreads)
 
 // S[b, v, :] = sum over the variable's edges of h[b, e, :] (in edge order);
 // thread = (variable, 8 columns), batch elements along y.
-template <typename T>
 __global__ void __launch_bounds__(kThreads)
-    k_mp_varsum(MpGraph g, const T* h, int64_t B, float* S) {
+    k_mp_varsum(MpGraph g, const u16* h, int64_t B, float* S) {
   for (int64_t t = blockIdx.x * int64_t(kThreads) + threadIdx.x; t < g.NV * 8;
        t += int64_t(gridDim.x) * kThreads) {
     const int64_t v = t >> 3;
     const int j0 = int(t & 7) * 8;
     const int32_t p0 = g.var_eptr[v], p1 = g.var_eptr[v + 1];
     for (int64_t b = blockIdx.y; b < B; b += gridDim.y) {
-      const T* hb = h + b * g.E * kH + j0;
+      const u16* hb = h + b * g.E * kH + j0;
       float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
       int32_t p = p0;
       for (; p + 4 <= p1; p += 4) {  // four rows in flight, summed in edge order
@@ -332,26 +320,6 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
-// Row `row` (< 64) of the layer input z for global row r, 8 values from
-// column 8c (c < 24), as BF16.
-__device__ __forceinline__ u32x4 z_chunk(const MpGraph& g, const u16* hin, const float* S,
-                                         int64_t r, int c) {
-  const int part = c >> 3, cc = (c & 7) * 8;
-  const int64_t b = r / g.E;
-  const int64_t e = r - b * g.E;
-  if (part == 0) return *reinterpret_cast<const u32x4*>(hin + r * kH + cc);
-  if (part == 2) return *reinterpret_cast<const u32x4*>(hin + (b * g.E + (e ^ 1)) * kH + cc);
-  const u32x4 hh = *reinterpret_cast<const u32x4*>(hin + r * kH + cc);
-  const float* s = S + (b * g.NV + g.edge_var[e]) * kH + cc;
-  u32x4 out;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    out[k] = pack_bf16(s[2 * k] - bf2f(u16(hh[k] & 0xffffu)),
-                       s[2 * k + 1] - bf2f(u16(hh[k] >> 16)));
-  }
-  return out;
-}
-
 constexpr int kZPad = kKZ + 8;  // LDS row pitch (elements) of 192-wide tiles
 constexpr int kHPad = kH + 8;   // LDS row pitch of 64-wide tiles
 
@@ -370,6 +338,26 @@ struct FwdRow {
   u32x4 h0, h1;  // activation columns 16q .. +15
   f32x4 s[4];    // variable-sum columns 16q .. +15
 };
+
+// Columns 16q .. +15 of the layer input z = [h, S_v - h, h_o] of tile row
+// `row`, and the same activation as the factor part of row ^ 1.
+__device__ __forceinline__ void fwd_row_to_lds(const FwdRow& x, u16* z, int row, int q) {
+  u16* zr = z + row * kZPad + 16 * q;
+  u16* zo = z + (row ^ 1) * kZPad + 2 * kH + 16 * q;
+  *reinterpret_cast<u32x4*>(zr) = x.h0;
+  *reinterpret_cast<u32x4*>(zr + 8) = x.h1;
+  *reinterpret_cast<u32x4*>(zo) = x.h0;
+  *reinterpret_cast<u32x4*>(zo + 8) = x.h1;
+  u32x4 d[2];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    const uint32_t hw = k < 4 ? x.h0[k] : x.h1[k - 4];
+    const float s0 = x.s[k >> 1][(2 * k) & 3], s1 = x.s[k >> 1][(2 * k + 1) & 3];
+    d[k >> 2][k & 3] = pack_bf16(s0 - bf2f(u16(hw & 0xffffu)), s1 - bf2f(u16(hw >> 16)));
+  }
+  *reinterpret_cast<u32x4*>(zr + kH) = d[0];
+  *reinterpret_cast<u32x4*>(zr + kH + 8) = d[1];
+}
 
 template <bool kHead>
 __global__ void __launch_bounds__(kFwdWaves * 64)
@@ -432,24 +420,7 @@ __global__ void __launch_bounds__(kFwdWaves * 64)
   bool okn = locate(tc + stride, &rn, &bn, &en);
   int32_t vn = okn ? g.edge_var[en] : 0;
   for (; tc < ntiles; tc += stride) {
-    // this tile's input rows into LDS
-    {
-      u16* zr = z + row * kZPad + 16 * q;
-      u16* zo = z + (row ^ 1) * kZPad + 2 * kH + 16 * q;
-      *reinterpret_cast<u32x4*>(zr) = cur.h0;
-      *reinterpret_cast<u32x4*>(zr + 8) = cur.h1;
-      *reinterpret_cast<u32x4*>(zo) = cur.h0;
-      *reinterpret_cast<u32x4*>(zo + 8) = cur.h1;
-      u32x4 d[2];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const uint32_t hw = k < 4 ? cur.h0[k] : cur.h1[k - 4];
-        const float s0 = cur.s[k >> 1][(2 * k) & 3], s1 = cur.s[k >> 1][(2 * k + 1) & 3];
-        d[k >> 2][k & 3] = pack_bf16(s0 - bf2f(u16(hw & 0xffffu)), s1 - bf2f(u16(hw >> 16)));
-      }
-      *reinterpret_cast<u32x4*>(zr + kH) = d[0];
-      *reinterpret_cast<u32x4*>(zr + kH + 8) = d[1];
-    }
+    fwd_row_to_lds(cur, z, row, q);
     const int64_t r_out = rc;
     const bool ok_out = okc;
     const int64_t b_out = bcur, e_out = ec;
@@ -709,120 +680,310 @@ __global__ void __launch_bounds__(kThreads)
   if (threadIdx.x == 0) loss_part[blockIdx.x] = red[0] * inv_n;
 }
 
-// g3 = dy w_h^T and per-workgroup partials of (dw_h, db_h).
+// One row's 16-byte piece of d h[pre-activation] in BF16: g * [h > 0].
+__device__ __forceinline__ u32x4 relu_grad8(const float* g, const u16* h) {
+  u32x4 out;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    out[k] = pack_bf16(bf2f(h[2 * k]) > 0.f ? g[2 * k] : 0.f,
+                       bf2f(h[2 * k + 1]) > 0.f ? g[2 * k + 1] : 0.f);
+  return out;
+}
+
+// dpre3 = (dy w_h^T) * [h3 > 0] in BF16, and per-workgroup partials of (dw_h,
+// db_h). Thread = (row, 8 columns), 32 rows a workgroup and step.
 __global__ void __launch_bounds__(kThreads)
-    k_mp_head_bwd(const u16* h3, const float* params, const float* dy, int64_t R, float* g,
+    k_mp_head_bwd(const u16* h3, const float* params, const float* dy, int64_t R, u16* dpre,
                   float* part) {
-  __shared__ float red[kThreads];
-  __shared__ float redb[4];
-  const int rg = threadIdx.x >> 6, j = threadIdx.x & 63;
-  const float wh = params[kOffWh + j];
-  float aw = 0.f, ab = 0.f;
-  for (int64_t r = blockIdx.x * 4 + rg; r < R; r += int64_t(gridDim.x) * 4) {
+  __shared__ float red[32][kH + 1];
+  const int rg = threadIdx.x >> 3, j0 = int(threadIdx.x & 7) * 8;
+  float wh[8], aw[8], ab = 0.f;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    wh[k] = params[kOffWh + j0 + k];
+    aw[k] = 0.f;
+  }
+  for (int64_t r = blockIdx.x * int64_t(32) + rg; r < R; r += int64_t(gridDim.x) * 32) {
     const float d = dy[r];
-    g[r * kH + j] = d * wh;
-    aw += d * bf2f(h3[r * kH + j]);
+    const u32x4 hv = *reinterpret_cast<const u32x4*>(h3 + r * kH + j0);
+    float g[8];
+    u16 h[8];
+    __builtin_memcpy(h, &hv, 16);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      g[k] = d * wh[k];
+      aw[k] += d * bf2f(h[k]);
+    }
+    *reinterpret_cast<u32x4*>(dpre + r * kH + j0) = relu_grad8(g, h);
     ab += d;
   }
-  red[threadIdx.x] = aw;
-  if (j == 0) redb[rg] = ab;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) red[rg][j0 + k] = aw[k];
+  if (j0 == 0) red[rg][kH] = ab;
   __syncthreads();
-  if (rg == 0) {
-    float s = red[j];
-    for (int q = 1; q < 4; ++q) s += red[q * 64 + j];
-    part[blockIdx.x * kHeadPart + j] = s;
-    if (j == 0) part[blockIdx.x * kHeadPart + kH] = ((redb[0] + redb[1]) + redb[2]) + redb[3];
+  if (threadIdx.x <= kH) {
+    float sum = 0.f;
+#pragma unroll
+    for (int q = 0; q < 32; ++q) sum += red[q][threadIdx.x];
+    part[blockIdx.x * kHeadPart + threadIdx.x] = sum;
   }
 }
 
-// Backward of one layer over tiles of 64 rows:
-//   dpre = g_out * [h_out > 0]
-//   dz = dpre W_l^T -> gin (self part), dV (variable-sum part), dF (factor part)
-//   dW_l += z^T dpre, db_l += sum(dpre)   (per-workgroup partials)
-__global__ void __launch_bounds__(kThreads)
-    k_mp_layer_bwd(MpGraph g, const u16* hin, const float* S, const u16* hout,
-                   const float* gout, const u16* wr, float* gin, float* dV, float* dF,
-                   float* part, int64_t R) {
-  __shared__ __attribute__((aligned(16))) u16 sW[kKZ * kHPad];       // W[i][j]
-  __shared__ __attribute__((aligned(16))) u16 sZt[kKZ * kHPad];      // z^T[i][row]
-  __shared__ __attribute__((aligned(16))) u16 sD[kTileRows * kHPad];  // dpre[row][j]
-  __shared__ __attribute__((aligned(16))) u16 sDt[kH * kHPad];        // dpre^T[j][row]
-  for (int q = threadIdx.x; q < kKZ * (kH / 8); q += kThreads) {
+// Backward of a layer z = [h, S_v - h, h_o], h_out = relu(z W + b), from
+// dpre = g_out * [h_out > 0] in BF16. dz = dpre W^T is linear, so the terms a
+// row's gradient collects from its variable's and its factor's other rows,
+//   g_in[e] = dpre_e Ws^T + sum_{e' at v, e' != e} dpre_e' Wv^T + dpre_o Wf^T,
+// are a product with [dpre_e, P_v - dpre_e, dpre_o] (P_v: the variable's sum of
+// dpre, k_mp_varsum), the forward's form: k_mp_layer_dgrad reads and writes one
+// row of BF16 per edge. (As dz parts in FP32, summed per variable and combined
+// in passes of their own, they were 480 MB of traffic a layer on 315,000 rows:
+// 325 us a layer with dW; now 32 + 11 here and 28 + 5 for dW, and the whole
+// step 1,287 -> 412.)
+//
+// P_v - dpre_e is an FP32 sum; it enters the BF16 product as three terms of 8
+// bits each, which hold all its 24 bits, so nothing of it is rounded away.
+//
+// Wavefronts work alone on tiles of 16 rows. A row-major row is an MFMA A
+// operand as it lies (lane l: row l % 16, 8 columns from 8 (l / 16)), so the
+// gathers go straight to registers, one tile ahead; only W and the result's
+// way back to rows use LDS. kInput: the masked result in FP32, for the input
+// layer's sums; else in BF16, dpre of the layer below.
+constexpr int kGPad = kH + 4;  // LDS row pitch (floats) of a result tile
+
+struct DgradRow {
+  u32x4 d[2];   // dpre columns 8g .. +7 and 32 + 8g .. +7
+  f32x4 p[4];   // variable-sum columns, the same
+  u32x4 h[2];   // layer input, row l / 4, columns 16 (l % 4) .. +15
+};
+
+template <bool kInput>
+__global__ void __launch_bounds__(kFwdWaves * 64)
+    k_mp_layer_dgrad(MpGraph g, const u16* dpre, const float* P, const u16* hin, const u16* wr,
+                     void* out, int64_t R) {
+  __shared__ __attribute__((aligned(16))) u16 sW[kKZ * kHPad];  // W[i][j]
+  __shared__ __attribute__((aligned(16))) float sG[kFwdWaves * kWaveRows * kGPad];
+  for (int q = threadIdx.x; q < kKZ * (kH / 8); q += kFwdWaves * 64) {
     const int i = q / (kH / 8), c = q % (kH / 8);
     *reinterpret_cast<u32x4*>(&sW[i * kHPad + c * 8]) =
         *reinterpret_cast<const u32x4*>(wr + i * kH + c * 8);
   }
-  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-  f32x4 accW[12];
+  __syncthreads();
+  const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int l = threadIdx.x & 63, row = l & 15, grp = l >> 4, orow = l >> 2, q = l & 3;
+  float* sg = sG + w * (kWaveRows * kGPad);
+  const int64_t ntiles = (R + kWaveRows - 1) / kWaveRows;
+  const int64_t stride = int64_t(gridDim.x) * kFwdWaves;
+  // the variable sum of this lane's row of tile t (null past the rows)
+  auto locate = [&](int64_t t) -> const float* {
+    const int64_t r0 = t * kWaveRows;
+    if (t >= ntiles || r0 + row >= R) return nullptr;
+    int64_t b = r0 / g.E, e = r0 - b * g.E + row;
+    while (e >= g.E) {
+      e -= g.E;
+      ++b;
+    }
+    return P + (b * g.NV + g.edge_var[e]) * kH;
+  };
+  auto gather = [&](int64_t t, const float* pv, DgradRow* x) {
+    const u32x4 none = {0u, 0u, 0u, 0u};
+    if (pv) {
+      const u16* d = dpre + (t * kWaveRows + row) * kH + 8 * grp;
 #pragma unroll
-  for (int q = 0; q < 12; ++q) accW[q] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float db = 0.f;
-  const int64_t ntiles = (R + kTileRows - 1) / kTileRows;
-  for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const int64_t r0 = tile * kTileRows;
-    __syncthreads();
-    for (int q = threadIdx.x; q < kTileRows * (kKZ / 8); q += kThreads) {
-      const int row = q % kTileRows, c = q / kTileRows;
-      const int64_t r = r0 + row;
-      u32x4 val = {0u, 0u, 0u, 0u};
-      if (r < R) val = z_chunk(g, hin, S, r, c);
+      for (int k = 0; k < 2; ++k) {
+        x->d[k] = *reinterpret_cast<const u32x4*>(d + 32 * k);
+        const f32x4* pp = reinterpret_cast<const f32x4*>(pv + 32 * k + 8 * grp);
+        x->p[2 * k] = pp[0];
+        x->p[2 * k + 1] = pp[1];
+      }
+    } else {
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        sZt[(c * 8 + 2 * k) * kHPad + row] = u16(val[k] & 0xffffu);
-        sZt[(c * 8 + 2 * k + 1) * kHPad + row] = u16(val[k] >> 16);
+      for (int k = 0; k < 2; ++k) {
+        x->d[k] = none;
+        x->p[2 * k] = x->p[2 * k + 1] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
     }
-    for (int q = threadIdx.x; q < kTileRows * kH; q += kThreads) {
-      const int row = q >> 6, j = q & 63;
-      const int64_t r = r0 + row;
-      u16 d = 0;
-      if (r < R && bf2f(hout[r * kH + j]) > 0.f) d = f2bf(gout[r * kH + j]);
-      sD[row * kHPad + j] = d;
-      sDt[j * kHPad + row] = d;
+    const int64_t ro = t * kWaveRows + orow;
+    x->h[0] = x->h[1] = none;
+    if (t < ntiles && ro < R) {
+      const u32x4* hp = reinterpret_cast<const u32x4*>(hin + ro * kH + 16 * q);
+      x->h[0] = hp[0];
+      x->h[1] = hp[1];
     }
-    __syncthreads();
-    // dz = dpre W^T: this wave's 16 rows x 192 columns
-    f32x4 acc[12];
+  };
+  int64_t t = int64_t(blockIdx.x) * kFwdWaves + w;
+  DgradRow cur;
+  gather(t, locate(t), &cur);
+  const float* pn = locate(t + stride);
+  for (; t < ntiles; t += stride) {
+    f32x4 acc[4];
 #pragma unroll
-    for (int nb = 0; nb < 12; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int n = 0; n < 4; ++n) acc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const DgradRow x = cur;
+    gather(t + stride, pn, &cur);  // next tile's rows, and the sum's address after that
+    pn = locate(t + 2 * stride);
 #pragma unroll
-    for (int ks = 0; ks < kH / 32; ++ks) {
-      const int kk = ks * 32 + 8 * (l >> 4);
-      const u32x4 a = *reinterpret_cast<const u32x4*>(&sD[(16 * w + (l & 15)) * kHPad + kk]);
-#pragma unroll
-      for (int nb = 0; nb < 12; ++nb) {
-        const u32x4 bb = *reinterpret_cast<const u32x4*>(&sW[(16 * nb + (l & 15)) * kHPad + kk]);
-        acc[nb] = mfma(a, bb, acc[nb]);
-      }
-    }
-#pragma unroll
-    for (int nb = 0; nb < 12; ++nb) {
-      const int col = 16 * nb + (l & 15);
-      float* dst = col < kH ? gin : (col < 2 * kH ? dV : dF);
-      const int cj = col & 63;
+    for (int k = 0; k < 2; ++k) {
+      u32x4 a[5];  // dpre_e, the three terms of P_v - dpre_e, dpre_o
+      a[0] = x.d[k];
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int64_t r = r0 + 16 * w + 4 * (l >> 4) + i;
-        if (r < R) dst[r * kH + cj] = acc[nb][i];
+        float s0 = x.p[2 * k + (i >> 1)][(2 * i) & 3] - bf2f(u16(x.d[k][i] & 0xffffu));
+        float s1 = x.p[2 * k + (i >> 1)][(2 * i + 1) & 3] - bf2f(u16(x.d[k][i] >> 16));
+#pragma unroll
+        for (int m = 1; m < 4; ++m) {
+          const uint32_t v = pack_bf16(s0, s1);
+          a[m][i] = v;
+          s0 -= bf2f(u16(v & 0xffffu));  // exact
+          s1 -= bf2f(u16(v >> 16));
+        }
+        // the factor's other edge is the neighbouring row, in the lane beside
+        a[4][i] = uint32_t(__builtin_amdgcn_mov_dpp(int(x.d[k][i]), 0xb1, 0xf, 0xf, false));
+      }
+#pragma unroll
+      for (int part = 0; part < 3; ++part)
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+          const u32x4 bb = *reinterpret_cast<const u32x4*>(
+              &sW[(kH * part + 16 * n + row) * kHPad + 32 * k + 8 * grp]);
+          if (part == 1) {
+            acc[n] = mfma(a[3], bb, acc[n]);
+            acc[n] = mfma(a[2], bb, acc[n]);
+            acc[n] = mfma(a[1], bb, acc[n]);
+          } else {
+            acc[n] = mfma(a[part == 0 ? 0 : 4], bb, acc[n]);
+          }
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sg[(4 * grp + i) * kGPad + 16 * n + row] = acc[n][i];
+    wave_lds_fence();
+    const int64_t ro = t * kWaveRows + orow;
+    if (ro < R) {
+      float gv[16];
+      u16 h[16];
+      __builtin_memcpy(h, x.h, 32);
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        *reinterpret_cast<f32x4*>(gv + 4 * k) =
+            *reinterpret_cast<const f32x4*>(sg + orow * kGPad + 16 * q + 4 * k);
+      if (kInput) {
+        f32x4* dst = reinterpret_cast<f32x4*>(static_cast<float*>(out) + ro * kH + 16 * q);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          f32x4 v;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = bf2f(h[4 * k + i]) > 0.f ? gv[4 * k + i] : 0.f;
+          dst[k] = v;
+        }
+      } else {
+        u32x4* dst = reinterpret_cast<u32x4*>(static_cast<u16*>(out) + ro * kH + 16 * q);
+        dst[0] = relu_grad8(gv, h);
+        dst[1] = relu_grad8(gv + 8, h + 8);
       }
     }
-    // dW += z^T dpre: this wave's 48 rows of W x 64 columns
+    wave_lds_fence();
+  }
+}
+
+// dW += z^T dpre and db += sum(dpre) over tiles of 64 rows (per-workgroup
+// partials). The contraction runs along the rows, so both operands are needed
+// column by column: the tiles lie in LDS as rows, written 16 bytes a lane, and
+// ds_read_b64_tr_b16 hands each lane four rows of one column. (Writing the
+// tiles transposed, 2 bytes a lane, and the tile's gathers and stores in one
+// chain between barriers made the whole backward layer 238 us on 315,000 rows.)
+// The next tile's gathers are in flight during this one's products. db is one
+// more product, with a row of ones. 28 us on 315,000 rows, 110 MB of gathers.
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+// A or B operand of rows row0 .. +31 and columns col0 .. +15 of an LDS tile:
+// lane l holds column col0 + l % 16, rows row0 + 8 (l / 16) .. +7.
+__device__ __forceinline__ u32x4 tile_columns(u16* tile, int pitch, int row0, int col0, int l) {
+  u16* p = tile + (row0 + 8 * (l >> 4) + ((l & 15) >> 2)) * pitch + col0 + 4 * (l & 3);
+  const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
+  const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(p + 4 * pitch));
+  u32x4 out;
+  __builtin_memcpy(&out, &lo, 8);
+  __builtin_memcpy(reinterpret_cast<char*>(&out) + 8, &hi, 8);
+  return out;
+}
+
+__global__ void __launch_bounds__(kThreads)
+    k_mp_layer_wgrad(MpGraph g, const u16* hin, const float* S, const u16* dpre, float* part,
+                     int64_t R) {
+  __shared__ __attribute__((aligned(16))) u16 sZ[kTileRows * kZPad];
+  __shared__ __attribute__((aligned(16))) u16 sD[kTileRows * kHPad];
+  const int w = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const int l = threadIdx.x & 63, row = threadIdx.x >> 2, q = threadIdx.x & 3;
+  f32x4 accW[12], accB = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < 12; ++k) accW[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint32_t one2 = pack_bf16(1.f, 1.f);
+  const u32x4 ones = {one2, one2, one2, one2};
+  const int64_t ntiles = (R + kTileRows - 1) / kTileRows;
+  const int64_t stride = gridDim.x;
+  auto locate = [&](int64_t t) -> const float* {
+    const int64_t r0 = t * kTileRows;
+    if (t >= ntiles || r0 + row >= R) return nullptr;
+    int64_t b = r0 / g.E, e = r0 - b * g.E + row;
+    while (e >= g.E) {
+      e -= g.E;
+      ++b;
+    }
+    return S + (b * g.NV + g.edge_var[e]) * kH;
+  };
+  struct Row {
+    FwdRow f;
+    u32x4 d0, d1;
+  };
+  auto gather = [&](int64_t t, const float* sv, Row* x) {
+    if (sv) {
+      const int64_t r = t * kTileRows + row;
+      const u32x4* hp = reinterpret_cast<const u32x4*>(hin + r * kH + 16 * q);
+      const u32x4* dp = reinterpret_cast<const u32x4*>(dpre + r * kH + 16 * q);
+      const f32x4* sp = reinterpret_cast<const f32x4*>(sv + 16 * q);
+      x->f.h0 = hp[0];
+      x->f.h1 = hp[1];
+      x->d0 = dp[0];
+      x->d1 = dp[1];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) x->f.s[k] = sp[k];
+    } else {
+      x->f.h0 = x->f.h1 = x->d0 = x->d1 = u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) x->f.s[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  int64_t t = blockIdx.x;
+  Row cur;
+  gather(t, locate(t), &cur);
+  const float* sn = locate(t + stride);
+  for (; t < ntiles; t += stride) {
+    fwd_row_to_lds(cur.f, sZ, row, q);
+    *reinterpret_cast<u32x4*>(sD + row * kHPad + 16 * q) = cur.d0;
+    *reinterpret_cast<u32x4*>(sD + row * kHPad + 16 * q + 8) = cur.d1;
+    gather(t + stride, sn, &cur);
+    sn = locate(t + 2 * stride);
+    __syncthreads();
 #pragma unroll
     for (int ks = 0; ks < kTileRows / 32; ++ks) {
-      const int kk = ks * 32 + 8 * (l >> 4);
+      u32x4 bb[4];
+#pragma unroll
+      for (int jb = 0; jb < 4; ++jb) bb[jb] = tile_columns(sD, kHPad, 32 * ks, 16 * jb, l);
 #pragma unroll
       for (int ib = 0; ib < 3; ++ib) {
-        const u32x4 a =
-            *reinterpret_cast<const u32x4*>(&sZt[(48 * w + 16 * ib + (l & 15)) * kHPad + kk]);
+        const u32x4 a = tile_columns(sZ, kZPad, 32 * ks, 48 * w + 16 * ib, l);
 #pragma unroll
-        for (int jb = 0; jb < 4; ++jb) {
-          const u32x4 bb = *reinterpret_cast<const u32x4*>(&sDt[(16 * jb + (l & 15)) * kHPad + kk]);
-          accW[ib * 4 + jb] = mfma(a, bb, accW[ib * 4 + jb]);
-        }
+        for (int jb = 0; jb < 4; ++jb) accW[ib * 4 + jb] = mfma(a, bb[jb], accW[ib * 4 + jb]);
       }
+      u32x4 mine = bb[0];  // this wave's 16 columns of db
+#pragma unroll
+      for (int jb = 1; jb < 4; ++jb) mine = w == jb ? bb[jb] : mine;
+      accB = mfma(ones, mine, accB);
     }
-    if (threadIdx.x < kH)
-      for (int row = 0; row < kTileRows; ++row) db += bf2f(sD[row * kHPad + threadIdx.x]);
+    __syncthreads();
   }
   float* p = part + int64_t(blockIdx.x) * kLayerPart;
 #pragma unroll
@@ -834,51 +995,64 @@ __global__ void __launch_bounds__(kThreads)
         const int wi = 48 * w + 16 * ib + 4 * (l >> 4) + i, wj = 16 * jb + (l & 15);
         p[wi * kH + wj] = accW[ib * 4 + jb][i];
       }
-  if (threadIdx.x < kH) p[kKZ * kH + threadIdx.x] = db;
+  if (l < 16) p[kKZ * kH + 16 * w + l] = accB[0];  // every row of the ones product is db
 }
 
-// gin[r] = d_self[r] + T[v(r)] - dV[r] + dF[o(r)]   (gin holds d_self on entry)
-__global__ void __launch_bounds__(kThreads)
-    k_mp_combine(MpGraph g, float* gin, const float* T, const float* dV, const float* dF,
-                 int64_t R) {
-  for (int64_t t = blockIdx.x * int64_t(kThreads) + threadIdx.x; t < R * kH;
-       t += int64_t(gridDim.x) * kThreads) {
-    const int64_t r = t >> 6;
-    const int j = int(t & 63);
-    const int64_t b = r / g.E, e = r - b * g.E;
-    const float tv = T[(b * g.NV + g.edge_var[e]) * kH + j];
-    gin[r * kH + j] =
-        ((gin[r * kH + j] + tv) - dV[r * kH + j]) + dF[(b * g.E + (e ^ 1)) * kH + j];
-  }
-}
-
-// dW0, db0 partials of the input layer (features recomputed).
+// dW0, db0 partials of the input layer, from dp = g0 * [h0 > 0] in FP32
+// (features recomputed, once per row: lane r of a wavefront's 64-row tile
+// leaves them in LDS, then lane j adds column j over the rows).
 __global__ void __launch_bounds__(kThreads)
     k_mp_embed_bwd(MpGraph g, const float* lp, int64_t lp_stride, const float* ev,
-                   int64_t ev_stride, const u16* h0, const float* g0, int64_t R, float* part) {
+                   int64_t ev_stride, const float* dp, int64_t R, float* part) {
+  __shared__ __attribute__((aligned(16))) float sx[kThreads / 64][kTileRows][kNin];
   __shared__ float red[kThreads * (kNin + 1)];
-  const int rg = threadIdx.x >> 6, j = threadIdx.x & 63;
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   float aw[kNin], ab = 0.f;
 #pragma unroll
   for (int k = 0; k < kNin; ++k) aw[k] = 0.f;
-  for (int64_t r = blockIdx.x * 4 + rg; r < R; r += int64_t(gridDim.x) * 4) {
-    const float dp = bf2f(h0[r * kH + j]) > 0.f ? g0[r * kH + j] : 0.f;
-    float x[kNin];
-    features(g, r, lp, lp_stride, ev, ev_stride, x);
+  const int64_t ntiles = (R + kTileRows - 1) / kTileRows;
+  for (int64_t t = blockIdx.x * int64_t(kThreads / 64) + w; t < ntiles;
+       t += int64_t(gridDim.x) * (kThreads / 64)) {
+    const int64_t r0 = t * kTileRows;
+    const int n = int(min(int64_t(kTileRows), R - r0));
+    if (l < n) {
+      float x[kNin];
+      features(g, r0 + l, lp, lp_stride, ev, ev_stride, x);
 #pragma unroll
-    for (int k = 0; k < kNin; ++k) aw[k] += x[k] * dp;
-    ab += dp;
+      for (int k = 0; k < kNin; ++k) sx[w][l][k] = x[k];
+    }
+    wave_lds_fence();
+    const float* d = dp + r0 * kH + l;
+    int i = 0;
+    for (; i + 8 <= n; i += 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = d[(i + u) * kH];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+#pragma unroll
+        for (int k = 0; k < kNin; ++k) aw[k] += sx[w][i + u][k] * v[u];
+        ab += v[u];
+      }
+    }
+    for (; i < n; ++i) {
+      const float v = d[i * kH];
+#pragma unroll
+      for (int k = 0; k < kNin; ++k) aw[k] += sx[w][i][k] * v;
+      ab += v;
+    }
+    wave_lds_fence();
   }
 #pragma unroll
   for (int k = 0; k < kNin; ++k) red[k * kThreads + threadIdx.x] = aw[k];
   red[kNin * kThreads + threadIdx.x] = ab;
   __syncthreads();
-  if (rg == 0) {
+  if (w == 0) {
     float* p = part + int64_t(blockIdx.x) * kEmbedPart;
     for (int k = 0; k <= kNin; ++k) {
-      const float* q = red + k * kThreads;
-      const float s = ((q[j] + q[64 + j]) + q[128 + j]) + q[192 + j];
-      p[(k < kNin ? k * kH : kNin * kH) + j] = s;
+      const float* c = red + k * kThreads;
+      const float sum = ((c[l] + c[64 + l]) + c[128 + l]) + c[192 + l];
+      p[(k < kNin ? k * kH : kNin * kH) + l] = sum;
     }
   }
 }
@@ -1072,7 +1246,7 @@ void forward(pgx_mpnn* n, const float* params, const float* lp, int64_t lp_strid
                      lp_stride, ev, ev_stride, B, static_cast<const int32_t*>(nullptr), h[0]);
   const unsigned lb = fwd_blocks(R);
   for (int l = 0; l < kLayers; ++l) {
-    hipLaunchKernelGGL(k_mp_varsum<u16>, item_batch_grid(g.NV * 8, B), dim3(kThreads), 0, s, g,
+    hipLaunchKernelGGL(k_mp_varsum, item_batch_grid(g.NV * 8, B), dim3(kThreads), 0, s, g,
                        static_cast<const u16*>(h[l]), B, S[l]);
     const float* bias = params + kOffL + l * kLayerSize + kKZ * kH;
     if (msgs && l == kLayers - 1)
@@ -1232,13 +1406,15 @@ int pgx_mpnn_grad(pgx_mpnn* n, const float* params, const float* lp, int64_t lp_
   if (!target || !grads || !loss) return set_error(PGX_EINVAL, "pgx_mpnn_grad: null argument");
   const int64_t B = batch, R = B * n->g.E, BV = B * n->g.NV;
   const unsigned lb = unsigned(std::min<int64_t>((R + kTileRows - 1) / kTileRows, kMaxLayerBlocks));
-  const unsigned hb_blocks = unsigned(std::min<int64_t>((R + 3) / 4, 1024));
+  const unsigned hb_blocks = unsigned(std::min<int64_t>((R + 31) / 32, 1024));
+  const unsigned eb_blocks = unsigned(std::min<int64_t>((R + 255) / 256, 1024));
   const unsigned loss_blocks = blocks_for(R);
   const size_t need = 2 * al256(size_t(kLayers) * kKZ * kH * 2) + 4 * al256(size_t(R) * kH * 2) +
-                      3 * al256(size_t(BV) * kH * 4) + 4 * al256(size_t(R) * kH * 4) +
+                      3 * al256(size_t(BV) * kH * 4) + 2 * al256(size_t(R) * kH * 2) +
+                      al256(size_t(R) * kH * 4) +
                       al256(size_t(R) * 4) + al256(size_t(BV) * kH * 4) +
                       al256(size_t(lb) * kLayerPart * 4) +
-                      al256(size_t(std::max<unsigned>(hb_blocks, loss_blocks)) *
+                      al256(size_t(std::max({hb_blocks, eb_blocks, loss_blocks})) *
                             std::max(kEmbedPart, kHeadPart) * 4) + 4096;
   if ((rc = grow(n, need))) return rc;
   Carve c{n->buf};
@@ -1248,14 +1424,13 @@ int pgx_mpnn_grad(pgx_mpnn* n, const float* params, const float* lp, int64_t lp_
   for (auto& x : h) x = c.take<u16>(size_t(R) * kH);
   float* S[3];
   for (auto& x : S) x = c.take<float>(size_t(BV) * kH);
-  float* ga = c.take<float>(size_t(R) * kH);
-  float* gb = c.take<float>(size_t(R) * kH);
-  float* dV = c.take<float>(size_t(R) * kH);
-  float* dF = c.take<float>(size_t(R) * kH);
+  u16* dcur = c.take<u16>(size_t(R) * kH);  // dpre of the layer at hand and the one below
+  u16* dnext = c.take<u16>(size_t(R) * kH);
+  float* dp0 = c.take<float>(size_t(R) * kH);
   float* dy = c.take<float>(size_t(R));
-  float* T = c.take<float>(size_t(BV) * kH);
+  float* P = c.take<float>(size_t(BV) * kH);
   float* lpart = c.take<float>(size_t(lb) * kLayerPart);
-  float* spart = c.take<float>(size_t(std::max<unsigned>(hb_blocks, loss_blocks)) *
+  float* spart = c.take<float>(size_t(std::max({hb_blocks, eb_blocks, loss_blocks})) *
                                std::max(kEmbedPart, kHeadPart));
   hipStream_t s = static_cast<hipStream_t>(stream);
   hipLaunchKernelGGL(k_mp_cast, dim3(blocks_for(kLayers * kKZ * kH)), dim3(kThreads), 0, s, params,
@@ -1266,25 +1441,31 @@ int pgx_mpnn_grad(pgx_mpnn* n, const float* params, const float* lp, int64_t lp_
                      static_cast<float*>(nullptr), int64_t(0), target, target_stride, dy, spart,
                      1.f / float(R));
   launch_reduce(spart, int32_t(loss_blocks), 1, 1, loss, s);
-  hipLaunchKernelGGL(k_mp_head_bwd, dim3(hb_blocks), dim3(kThreads), 0, s, h[3], params, dy, R, ga,
+  hipLaunchKernelGGL(k_mp_head_bwd, dim3(hb_blocks), dim3(kThreads), 0, s, h[3], params, dy, R, dcur,
                      spart);
   launch_reduce(spart, int32_t(hb_blocks), kHeadPart, kHeadPart, grads + kOffWh, s);
-  float* gout = ga;
-  float* gin = gb;
+  const unsigned db = fwd_blocks(R);
   for (int l = kLayers - 1; l >= 0; --l) {
-    hipLaunchKernelGGL(k_mp_layer_bwd, dim3(lb), dim3(kThreads), 0, s, n->g, h[l], S[l], h[l + 1],
-                       gout, wr + l * kKZ * kH, gin, dV, dF, lpart, R);
+    hipLaunchKernelGGL(k_mp_layer_wgrad, dim3(lb), dim3(kThreads), 0, s, n->g,
+                       static_cast<const u16*>(h[l]), static_cast<const float*>(S[l]),
+                       static_cast<const u16*>(dcur), lpart, R);
     launch_reduce(lpart, int32_t(lb), kLayerPart, kLayerPart, grads + kOffL + l * kLayerSize, s);
-    hipLaunchKernelGGL(k_mp_varsum<float>, item_batch_grid(n->g.NV * 8, B), dim3(kThreads), 0, s,
-                       n->g, static_cast<const float*>(dV), B, T);
-    hipLaunchKernelGGL(k_mp_combine, dim3(blocks_for(R * kH)), dim3(kThreads), 0, s, n->g, gin,
-                       static_cast<const float*>(T), static_cast<const float*>(dV),
-                       static_cast<const float*>(dF), R);
-    std::swap(gout, gin);
+    hipLaunchKernelGGL(k_mp_varsum, item_batch_grid(n->g.NV * 8, B), dim3(kThreads), 0, s, n->g,
+                       static_cast<const u16*>(dcur), B, P);
+    const u16* wl = wr + l * kKZ * kH;
+    if (l > 0)
+      hipLaunchKernelGGL(k_mp_layer_dgrad<false>, dim3(db), dim3(kFwdWaves * 64), 0, s, n->g,
+                         static_cast<const u16*>(dcur), static_cast<const float*>(P),
+                         static_cast<const u16*>(h[l]), wl, static_cast<void*>(dnext), R);
+    else
+      hipLaunchKernelGGL(k_mp_layer_dgrad<true>, dim3(db), dim3(kFwdWaves * 64), 0, s, n->g,
+                         static_cast<const u16*>(dcur), static_cast<const float*>(P),
+                         static_cast<const u16*>(h[l]), wl, static_cast<void*>(dp0), R);
+    std::swap(dcur, dnext);
   }
-  hipLaunchKernelGGL(k_mp_embed_bwd, dim3(hb_blocks), dim3(kThreads), 0, s, n->g, lp, lp_stride,
-                     ev, ev_stride, h[0], gout, R, spart);
-  launch_reduce(spart, int32_t(hb_blocks), kEmbedPart, kEmbedPart, grads + kOffW0, s);
+  hipLaunchKernelGGL(k_mp_embed_bwd, dim3(eb_blocks), dim3(kThreads), 0, s, n->g, lp, lp_stride,
+                     ev, ev_stride, static_cast<const float*>(dp0), R, spart);
+  launch_reduce(spart, int32_t(eb_blocks), kEmbedPart, kEmbedPart, grads + kOffW0, s);
   PGX_HIP(hipGetLastError());
   return PGX_OK;
 }

@@ -263,6 +263,42 @@ def test_gpu_gradients_match_oracle(gpu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("num,pairs,batch_size", [
+    (2, "pair", 1),     # 2 rows: most of a tile empty
+    (2, "pair", 37),    # variables' rows cross tiles of 16 and 64
+    (21, "star", 3),    # 20 edges on a variable, 120 rows
+    (9, "chain", 8),    # 128 rows: two whole tiles of 64
+    (9, "chain", 9),    # and 16 rows more
+])
+def test_gpu_gradients_at_tile_edges(gpu, num, pairs, batch_size):
+  """Backward tiles of 16 and 64 rows that are empty, full and cut by a batch
+  element's end, against the oracle; the bar of the test above."""
+  import torch
+  from pgmax_amd import engine, warmstart
+  pairs = {"pair": [[0, 1]], "star": [[0, i] for i in range(1, num)],
+           "chain": [[i, i + 1] for i in range(num - 1)]}[pairs]
+  w = batch.pairwise_wiring(num, 2, np.array(pairs), full_tables=True)
+  rng = np.random.default_rng(num + batch_size)
+  j = rng.normal(size=(batch_size, len(pairs)))
+  lp = np.stack([j, -j, -j, j], -1).reshape(batch_size, -1).astype(np.float32)
+  ev = rng.normal(0, 0.5, size=(batch_size, 2 * num)).astype(np.float32)
+  target = np.stack([omp.messages_from_ratio(rng.normal(size=2 * len(pairs)))
+                     for _ in range(batch_size)]).astype(np.float32)
+  graph = engine.Graph(w.to_engine_wiring())
+  flat = omp.to_flat(omp.init_params(5))
+  net = warmstart.WarmStart(graph, params=(flat + 0.02 * rng.normal(size=flat.size)).astype(
+      np.float32))
+  loss, grads = net.loss_and_grad(*(torch.as_tensor(x) for x in (lp, ev, target)))
+  got = omp.from_flat(grads.cpu().numpy())
+  _, want, loss_ref = _oracle_rows(w, lp, ev, omp.from_flat(net.params.cpu().numpy()), target)
+  assert float(loss.cpu()) == pytest.approx(loss_ref, rel=1e-6)
+  for k in want:
+    assert np.linalg.norm(got[k] - want[k]) <= 7e-5 * np.linalg.norm(want[k]) + 1e-12, k
+  net.close()
+  graph.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("side,copies", [(3, 2), (5, 64), (33, 64), (40, 128)])
 def test_gpu_gradients_of_repeated_graph(gpu, side, copies):
   """A batch of 2^k copies of one graph has its loss and gradients: the mean
