@@ -416,6 +416,15 @@ int pgx_graph_create(const pgx_wiring* wiring, pgx_graph** out) {
     }
     d.var_pos4 = reinterpret_cast<const int4*>(vp4);
   }
+  if (!P.var_pos2.empty()) {
+    int32_t* vp2;
+    if ((rc = up(P.var_pos2, &vp2))) {
+      pgx_graph_destroy(g);
+      return rc;
+    }
+    d.var_pos2 = reinterpret_cast<const int2*>(vp2);
+  }
+  d.binary_vars = P.binary_vars ? 1 : 0;
   if (!P.edge_pos4.empty()) {
     int32_t* ep4;
     if ((rc = up(P.edge_pos4, &ep4))) {
@@ -1340,19 +1349,23 @@ int pgx_get_beliefs(pgx_graph* g, const float* ev, int64_t ev_stride, const floa
                   aligned(beliefs, 8))
                      ? 1
                      : 0;
-  // the caller's messages are in the reference layout
+  // the caller's messages are in the reference layout, two floats each
   DevGraph dref = g->dev;
-  dref.var_adj_es = dref.var_adj_es_ref;
-  // the row split and chunk strides hold for engine positions only: every
-  // chunk in order, positions loaded
-  dref.heavy_col = nullptr;
-  dref.col_desc = nullptr;
-  dref.chunk_desc = g->chunk_desc_ref;
-  dref.heavy_chunk_stride = g->zero_strides;
-  dref.num_heavy_col = dref.num_heavy_chunks;
-  dref.num_heavy_row = 0;
-  dref.var_pos4 = nullptr;  // engine positions
-  dref.edge_pos4 = nullptr;
+  dref.packed = 0;
+  if (dref.perm) {
+    // the descriptors hold engine positions: every chunk in order, positions
+    // loaded
+    dref.var_adj_es = dref.var_adj_es_ref;
+    dref.heavy_col = nullptr;
+    dref.col_desc = nullptr;
+    dref.chunk_desc = g->chunk_desc_ref;
+    dref.heavy_chunk_stride = g->zero_strides;
+    dref.num_heavy_col = dref.num_heavy_chunks;
+    dref.num_heavy_row = 0;
+    dref.var_pos4 = nullptr;
+    dref.var_pos2 = nullptr;
+    dref.edge_pos4 = nullptr;
+  }
   launch_var_phase(dref, ftov, ftov_stride, ev, ev_stride, beliefs, g->bscratch, batch, s);
   PGX_HIP(hipGetLastError());
   return PGX_OK;

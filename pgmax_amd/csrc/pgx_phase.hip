@@ -63,6 +63,10 @@ __global__ void __launch_bounds__(256)
 // row chunk per 8 lanes, then one variable of more than kThreadStates states
 // per 16 lanes: one thread walking 16 states of one variable after the other
 // took 22.7 us an iteration on 45 x 61 variables, the lane groups take 3.9.
+// kBinary: graphs of binary variables, whose states need no index loads and
+// whose sums few registers (1.4 million variables and 5.3 million edges of six
+// deconvolution images: 49.5 us in the general form, now 40.8).
+template <bool kBinary>
 __global__ void __launch_bounds__(kPhaseThreads)
     k_var_phase(DevGraph g, const float* m, int64_t m_stride, const float* ev,
                 int64_t ev_stride, float* out, float* partial, int32_t light_blocks,
@@ -73,25 +77,36 @@ __global__ void __launch_bounds__(kPhaseThreads)
   const int32_t blk_x = int32_t(bx);
   if (blk_x < light_blocks) {
     const int32_t v = blk_x * kPhaseThreads + threadIdx.x;
-    if (v < g.num_vars)
-      var_sums(g, v, m + b * m_stride, ev + b * ev_stride, out + b * g.num_vs, true);
+    if (v < g.num_vars) {
+      if constexpr (kBinary)
+        var_sums_binary(g, v, m + b * m_stride, ev + b * ev_stride, out + b * g.num_vs);
+      else
+        var_sums(g, v, m + b * m_stride, ev + b * ev_stride, out + b * g.num_vs, true);
+    }
     return;
   }
   if (blk_x < light_blocks + col_blocks) {
     const int32_t i = (blk_x - light_blocks) * kPhaseThreads + threadIdx.x;
-    if (i < g.num_heavy_col)
-      heavy_chunk_d(g, g.col_desc ? g.col_desc[i] : g.chunk_desc[i], m + b * m_stride,
-                    partial + b * g.partial_size);
+    if (i < g.num_heavy_col) {
+      const int4 d = g.col_desc ? g.col_desc[i] : g.chunk_desc[i];
+      float* part = partial + b * g.partial_size;
+      if constexpr (kBinary)
+        heavy_chunk_t<2>(g, d.x, d.x + (d.y & 0xff), 2, m + b * m_stride, part + d.z, d.w);
+      else
+        heavy_chunk_d(g, d, m + b * m_stride, part);
+    }
     return;
   }
-  if (blk_x >= light_blocks + col_blocks + row_blocks) {
-    const int32_t i = (blk_x - light_blocks - col_blocks - row_blocks) *
-                          (kPhaseThreads / kWideVarLanes) +
-                      int32_t(threadIdx.x) / kWideVarLanes;
-    if (i < g.num_wide)
-      wide_var_sums(g, g.wide_desc[i], int32_t(threadIdx.x) % kWideVarLanes, m + b * m_stride,
-                    ev + b * ev_stride, out + b * g.num_vs);
-    return;
+  if constexpr (!kBinary) {
+    if (blk_x >= light_blocks + col_blocks + row_blocks) {
+      const int32_t i = (blk_x - light_blocks - col_blocks - row_blocks) *
+                            (kPhaseThreads / kWideVarLanes) +
+                        int32_t(threadIdx.x) / kWideVarLanes;
+      if (i < g.num_wide)
+        wide_var_sums(g, g.wide_desc[i], int32_t(threadIdx.x) % kWideVarLanes, m + b * m_stride,
+                      ev + b * ev_stride, out + b * g.num_vs);
+      return;
+    }
   }
   __shared__ float stage[(kPhaseThreads / kRowLanes) * kRowStride];
   const int32_t grp = int32_t(threadIdx.x) / kRowLanes;
@@ -141,7 +156,7 @@ __device__ __forceinline__ void fac_phase_body(const DevGraph& g, const Tile* ti
       const int32_t i = tile.i0 + int32_t(threadIdx.x) / 64;
       if (i < tile.i1)
         logical_factor_wave<EngineIO>(g, blk.f0 + i, blk.off, io, t, true, dl,
-                                      int32_t(threadIdx.x) % 64);
+                                      int32_t(threadIdx.x) % 64, (blk.pad[0] & 64) != 0);
       block_delta_store<kPhaseThreads>(dl, delta_dst<kConv>(g, r, blk, b, it));
       return;
     }
@@ -150,6 +165,16 @@ __device__ __forceinline__ void fac_phase_body(const DevGraph& g, const Tile* ti
       if (i < tile.i1)
         logical_factor_wide<EngineIO>(g, blk.f0 + i, blk.off, io, t, true, dl,
                                       int32_t(threadIdx.x) % kWideLanes);
+      block_delta_store<kPhaseThreads>(dl, delta_dst<kConv>(g, r, blk, b, it));
+      return;
+    }
+    // factors of few parents, all as many: no factor or position loads (1.3
+    // million AND factors of two parents: 45.6 us an iteration, now 41.5)
+    if ((blk.pad[0] & 64) && blk.nv > 0 && blk.nv <= kSmallParents + 1) {
+      const int32_t i = tile.i0 + threadIdx.x;
+      if (i < tile.i1)
+        logical_small<EngineIO>(g, blk.e0 + blk.nv * i, blk.nv - 1, blk.off, io, t, true, dl,
+                                blk.es0 + 2 * blk.nv * i);
       block_delta_store<kPhaseThreads>(dl, delta_dst<kConv>(g, r, blk, b, it));
       return;
     }
@@ -327,7 +352,10 @@ __global__ void __launch_bounds__(kPhaseThreads)
 template <bool kT0, int KIND, bool kConv>
 __global__ void __launch_bounds__(kPhaseThreads)
     k_fac_phase(DevGraph g, const Tile* tiles, RunBufs r, int32_t it) {
-  if (!kT0 && r.t == 1.f)
+  // (t as a constant at T = 0 too: the logical updates leave out the rest)
+  if (kT0)
+    fac_phase_body<kT0, KIND, kConv>(g, tiles, r, it, 0.f);
+  else if (r.t == 1.f)
     fac_phase_body<kT0, KIND, kConv>(g, tiles, r, it, 1.f);
   else
     fac_phase_body<kT0, KIND, kConv>(g, tiles, r, it, r.t);
@@ -498,8 +526,12 @@ void launch_var_phase(const DevGraph& d, const float* m, int64_t m_stride, const
   const KernelClock off;
   const KernelClock& c = clk ? *clk : off;
   c.run(PGX_KERNEL_VAR_PHASE, [&] {
-    hipLaunchKernelGGL(k_var_phase, vgrid, dim3(kPhaseThreads), 0, s, d, m, m_stride, ev,
-                       ev_stride, out, partial, light_blocks, col_blocks, row_blocks, xcd);
+    if (d.binary_vars)
+      hipLaunchKernelGGL((k_var_phase<true>), vgrid, dim3(kPhaseThreads), 0, s, d, m, m_stride,
+                         ev, ev_stride, out, partial, light_blocks, col_blocks, row_blocks, xcd);
+    else
+      hipLaunchKernelGGL((k_var_phase<false>), vgrid, dim3(kPhaseThreads), 0, s, d, m, m_stride,
+                         ev, ev_stride, out, partial, light_blocks, col_blocks, row_blocks, xcd);
   });
   if (d.num_vh_groups > 0)
     c.run(PGX_KERNEL_VAR_COMBINE, [&] {

@@ -518,9 +518,21 @@ int build_plan(const pgx_wiring& w, Plan* P, std::string* err, int64_t merge_bel
     if (b.kind == kOr || b.kind == kAnd) {
       // factors of more than one run of parents go to lane groups (all of
       // the block's factors have at most kWideRuns runs)
-      int32_t maxp = 0;
-      for (int32_t i = 0; i < b.count; ++i)
-        maxp = std::max(maxp, P->fac_e0[b.f0 + i + 1] - P->fac_e0[b.f0 + i] - 1);
+      int32_t maxp = 0, minp = b.count > 0 ? E : 0;
+      for (int32_t i = 0; i < b.count; ++i) {
+        const int32_t np = P->fac_e0[b.f0 + i + 1] - P->fac_e0[b.f0 + i] - 1;
+        maxp = std::max(maxp, np);
+        minp = std::min(minp, np);
+      }
+      const int32_t e1 = P->fac_e0[b.f0 + b.count];
+      bool binary = true;
+      for (int32_t e = b.e0; e < e1 && binary; ++e)
+        binary = P->edge_es0[e] == b.es0 + 2 * (e - b.e0) &&
+                 P->edge_es0[e + 1] == P->edge_es0[e] + 2;
+      if (binary) {
+        b.pad[0] |= 64;
+        b.nv = maxp == minp ? maxp + 1 : 0;
+      }
       // (one wavefront per factor when all have at most 256 parents)
       if (maxp > kVarChunk && maxp <= kWaveLogicalParents) b.pad[0] |= 16;
       else if (maxp > kVarChunk && maxp <= kWideRuns * kVarChunk) b.pad[0] |= 4;
@@ -555,6 +567,19 @@ int build_plan(const pgx_wiring& w, Plan* P, std::string* err, int64_t merge_bel
         for (int k = 0; k < 4; ++k)
           P->edge_pos4[size_t(e) * 4 + k] = P->var_pos4[size_t(edge_var[e]) * 4 + k];
     }
+  }
+
+  P->binary_vars = NV > 0 && int64_t(Vs) == int64_t(NV) * 2;
+  int32_t light = 0;  // most edges of a variable with a descriptor
+  for (int32_t v = 0; v < NV; ++v) {
+    P->binary_vars = P->binary_vars && P->var_vs0[v] == 2 * v;
+    const int32_t deg = P->var_eptr[v + 1] - P->var_eptr[v];
+    if (deg <= 4) light = std::max(light, deg);
+  }
+  if (P->binary_vars && light <= 2 && !P->pairwise_only && !P->var_pos4.empty()) {
+    P->var_pos2.resize(size_t(NV) * 2);
+    for (int32_t v = 0; v < NV; ++v)
+      for (int k = 0; k < 2; ++k) P->var_pos2[size_t(v) * 2 + k] = P->var_pos4[size_t(v) * 4 + k];
   }
 
   P->packable = !P->var_pos4.empty() && !P->perm.empty() && P->even2 && P->max_degree <= 4 &&
@@ -620,7 +645,10 @@ int build_plan(const pgx_wiring& w, Plan* P, std::string* err, int64_t merge_bel
     const int32_t a = P->var_eptr[v] + k * kVarChunk;
     const int32_t z = std::min(a + kVarChunk, P->var_eptr[v + 1]);
     bool row = P->var_vs0[v + 1] - P->var_vs0[v] == 2;
-    for (int32_t p = a; row && p + 1 < z; ++p) row = P->var_adj_es[p + 1] == P->var_adj_es[p] + 2;
+    const int32_t step = z - a > 1 ? P->var_adj_es[a + 1] - P->var_adj_es[a] : 2;
+    row = row && step > 0 && step <= kRowStep;
+    for (int32_t p = a; row && p + 1 < z; ++p)
+      row = P->var_adj_es[p + 1] == P->var_adj_es[p] + step;
     (row ? P->heavy_row_chunks : P->heavy_col_chunks).push_back(hc);
     int32_t stride = 0;
     if (z - a == kVarChunk) {
@@ -641,7 +669,10 @@ int build_plan(const pgx_wiring& w, Plan* P, std::string* err, int64_t merge_bel
       const int32_t len = std::min(a + kVarChunk, P->var_eptr[v + 1]) - a;
       return std::array<int32_t, 4>{row ? P->var_adj_es[a] : a, len | (ns << 8),
                                     P->heavy_pofs[h] + k * ns,
-                                    (row || ref) ? 0 : P->heavy_chunk_stride[hc]};
+                                    row   ? (len > 1 ? P->var_adj_es[a + 1] - P->var_adj_es[a]
+                                                     : 2)
+                                    : ref ? 0
+                                          : P->heavy_chunk_stride[hc]};
     };
     for (int32_t h = 0; h < int32_t(P->heavy_vars.size()); ++h) {
       const int32_t v = P->heavy_vars[h];

@@ -32,7 +32,7 @@ struct Block {
   int32_t count;   // number of factors
   int32_t e0;      // first edge of factor f0
   int32_t es0;     // first edge state of factor f0
-  int32_t nv;      // Enum: edges per factor
+  int32_t nv;      // edges per factor (OR/AND: 0 unless bit 6 and the same for all)
   int32_t esf;     // Enum: edge states per factor
   int32_t c0;      // Enum: absolute log-potential index of factor f0, config 0
   int32_t nc;      // Enum: configs per factor
@@ -45,7 +45,9 @@ struct Block {
                    // bit 3: general Enum block run by one wavefront per factor,
                    // bit 4: OR/AND block run by one wavefront per factor,
                    // bit 5: general Enum block of full pairwise tables (s0 x s1,
-                   // row-major) run with one lane per edge state (pair_wide)
+                   // row-major) run with one lane per edge state (pair_wide),
+                   // bit 6: OR/AND block of binary edges (edge k of a factor at
+                   // its first edge state + 2k); nv > 0: edges of every factor
 };
 
 // Long sums (incident edges of a variable, parents of a logical factor) run
@@ -63,6 +65,9 @@ constexpr int32_t kWaveMaxStates = 256;
 // factor, 64 / (s0 + s1) factors per wavefront, their summaries in the
 // wavefront's LDS.
 constexpr int32_t kPairWideStates = 64;  // most edge states of such a factor
+// Positions of a row chunk's edges are at most this many floats apart (the
+// edges of one slot of consecutive factors of up to four binary edges).
+constexpr int32_t kRowStep = 8;
 // Variables of more than kThreadStates states are summed by a lane group each.
 constexpr int32_t kThreadStates = 8;
 constexpr int64_t kPos4MaxBytes = int64_t(1) << 30;        // per-variable descriptors
@@ -107,13 +112,14 @@ struct Plan {
   // groups of kVarChunk: heavy_gpofs[h] is the first group-sum slot (after
   // all chunk slots) or -1; (vh_group_h, vh_group_j) enumerate the groups.
   // Chunks split for the per-phase variable kernel: "row" chunks hold a
-  // binary variable's 32 edges at consecutive positions (one 8-lane group
-  // reads them together), "col" chunks the rest (one thread each).
+  // binary variable's edges at evenly spaced positions at most kRowStep apart
+  // (one 8-lane group reads them together), "col" chunks the rest (one thread
+  // each).
   std::vector<int32_t> heavy_chunk_stride;  // [NHC] position step of a full chunk whose
                                             // edges are evenly spaced, else 0
   // Chunk descriptors, 4 ints each, so a kernel reads one record per chunk:
   // [first adjacency index (row chunks: first engine position), len | ns << 8,
-  //  partial-sum slot, position step or 0]. chunk_desc in chunk order,
+  //  partial-sum slot, position step (col chunks: or 0)]. chunk_desc in chunk order,
   // chunk_desc_ref the same with step 0 (reference layout), col_desc /
   // row_desc in the order of heavy_col_chunks / heavy_row_chunks.
   std::vector<int32_t> chunk_desc, chunk_desc_ref, col_desc, row_desc;
@@ -142,6 +148,10 @@ struct Plan {
   // the entry of each edge's variable (graphs whose factor side recomputes
   // variable sums). Empty past kPos4MaxBytes / kEdgePos4MaxBytes.
   std::vector<int32_t> var_pos4, edge_pos4;
+  // Every variable binary, its states at 2v. var_pos2 (then, when no variable
+  // has 3 or 4 edges): var_pos4's entries cut to two.
+  bool binary_vars = false;
+  std::vector<int32_t> var_pos2;
   // Every factor a planar 2x2 Enum factor and every variable binary with at
   // most 4 edges: the per-phase shape may keep one float per message.
   bool packable = false;

@@ -242,3 +242,41 @@ def test_patches_match_oracle(gpu, kind, temperature, iters):
     for o, od in ((out, d), (auto, auto_d)):
       np.testing.assert_array_equal(_np(o)[b], ref)
       np.testing.assert_array_equal(_np(od)[b], ref_d)
+
+
+@pytest.mark.parametrize("kind", ["parents 1", "parents 2", "parents 3", "mixed", "wave"])
+@pytest.mark.parametrize("logical", ["or", "and"])
+@pytest.mark.parametrize("temperature", [0.0, 0.7])
+def test_logical_blocks_match_oracle(gpu, kind, logical, temperature):
+  """OR / AND blocks whose factors all have as many parents and whose do not,
+  and the row chunks of a variable that is the same slot of 41 and of 65
+  consecutive factors (positions 4, 6 and 8 floats apart, whole and partial
+  chunks, a lone edge), in the per-phase and the automatic shape."""
+  group = {"or": fgroup.ORFactorGroup, "and": fgroup.ANDFactorGroup}[logical]
+  rng = np.random.default_rng(23)
+  v = vgroup.NDVarArray(num_states=2, shape=(700,))
+  if kind == "wave":
+    facs = [[v[i] for i in rng.choice(700, size=n + 1, replace=False)]
+            for n in (33, 64, 128, 255, 256)]
+  else:
+    sizes = [2] * 106 if kind == "mixed" else [int(kind[-1])] * 106
+    if kind == "mixed":
+      sizes[3], sizes[50], sizes[90] = 1, 3, 3
+    rest, facs = iter(range(2, 700)), []
+    for i, n in enumerate(sizes):  # variable 0 in 41 factors, then variable 1 in 65
+      facs.append([v[0] if i < 41 else v[1]] + [v[next(rest)] for _ in range(n)])
+  fg = fgraph.FactorGraph(variable_groups=v)
+  fg.add_factors(group(variables_for_factors=facs))
+  bp = infer.BP(fg.bp_state, temperature=temperature)
+  graph = lbp.graph_from_context(bp.context)
+  ev = rng.normal(size=1400).astype(np.float32)
+  ft = rng.normal(size=bp.init().ftov_msgs.shape[0]).astype(np.float32)
+  lp = np.zeros((0,), np.float32)
+  ref, ref_d = lbp.run_with_diffs(graph, lp, ft, ev, 5, 0.5, temperature)
+  for mode in (0, 2):
+    _lib.set_option("mode", mode)
+    out, d = bp.run_with_diffs(infer.BPArrays(log_potentials=lp, ftov_msgs=ft, evidence=ev), 5)
+    np.testing.assert_array_equal(_np(out.ftov_msgs), ref)
+    np.testing.assert_array_equal(_np(d), ref_d)
+  np.testing.assert_array_equal(_np(bp.context.get_flat_beliefs(out)),
+                                lbp.get_flat_beliefs(graph, ref, ev))
