@@ -37,7 +37,6 @@ struct DevGraph {
   const int32_t* heavy_pofs;
   const int32_t* heavy_chunk_var;
   const int32_t* heavy_chunk_k;
-  const int32_t* heavy_gpofs;  // group-sum slots of very heavy variables, or -1
   const int32_t* heavy_chunk_stride;  // evenly spaced full chunks: position step, else 0
   const int32_t* heavy_col;    // chunks summed one per thread (null: all, in order)
   const int32_t* heavy_row;    // chunks of consecutive binary edges, one per 8-lane group
@@ -48,9 +47,8 @@ struct DevGraph {
   const int4* heavy_desc;      // per heavy variable -- see Plan::heavy_desc
   const int4* wide_desc;       // per variable of many states -- see Plan::wide_desc
   int32_t num_wide;
-  const int32_t* vh_group_h;
-  const int32_t* vh_group_j;
-  int32_t num_vh_groups;
+  const int32_t* heavy_groups;  // heavy variables of more than kVarChunk chunks
+  int32_t num_heavy_groups;
   const int32_t* perm;            // engine position of each reference edge state, or null
   const int32_t* var_adj_es_ref;  // var_adj_es in the reference layout
   const int32_t* edge_var;
@@ -2172,12 +2170,11 @@ __device__ __forceinline__ void chunk_total2(const float* part, int32_t nch, flo
 }
 
 // Heavy variable h: chunk sums in order, then + evidence.
+// chunk sums are added in groups of kVarChunk (each from 0), then the group
+// sums in order (from 0), then the evidence
 __device__ __forceinline__ void heavy_combine(const DevGraph& g, int32_t h,
                                              const float* partial, const float* ev,
-                                             float* out, bool groups_ready = false) {
-  // chunk sums are added in groups of kVarChunk (each from 0), then the
-  // group sums in order (from 0), then the evidence; with groups_ready the
-  // group sums were written by k_var_groups
+                                             float* out) {
   const int4 hd = g.heavy_desc[h];
   const int32_t vs0 = hd.x, ns = hd.y >> 16;
   const int32_t nch = hd.y & 0xffff;
@@ -2185,29 +2182,57 @@ __device__ __forceinline__ void heavy_combine(const DevGraph& g, int32_t h,
   const float* part = partial + hd.z;
   if (ns == 2) {
     float t0, t1;
-    if (groups_ready && ng > 1) {
-      sum_range2(partial + hd.w, 0, ng, t0, t1);
-    } else {
-      chunk_total2(part, nch, t0, t1);
-    }
+    chunk_total2(part, nch, t0, t1);
     out[vs0] = t0 + ev[vs0];
     out[vs0 + 1] = t1 + ev[vs0 + 1];
     return;
   }
   for (int32_t s = 0; s < ns; ++s) {
     float tot = 0.f;
-    if (groups_ready && ng > 1) {
-      const float* gp = partial + hd.w;
-      for (int32_t j = 0; j < ng; ++j) tot += gp[j * ns + s];
-    } else {
-      for (int32_t j = 0; j < ng; ++j) {
-        float gs = 0.f;
-        const int32_t k1 = min(nch, (j + 1) * kVarChunk);
-        for (int32_t k = j * kVarChunk; k < k1; ++k) gs += part[k * ns + s];
-        tot += gs;
-      }
+    for (int32_t j = 0; j < ng; ++j) {
+      float gs = 0.f;
+      const int32_t k1 = min(nch, (j + 1) * kVarChunk);
+      for (int32_t k = j * kVarChunk; k < k1; ++k) gs += part[k * ns + s];
+      tot += gs;
     }
     out[vs0 + s] = tot + ev[vs0 + s];
+  }
+}
+
+// heavy_combine of a variable of several groups by one wavefront: a lane sums
+// a group, the group sums are added in order. Every lane must call it.
+__device__ __forceinline__ void heavy_combine_wave(const DevGraph& g, int32_t h, int32_t lane,
+                                                   const float* partial, const float* ev,
+                                                   float* out) {
+  const int4 hd = g.heavy_desc[h];
+  const int32_t vs0 = hd.x, ns = hd.y >> 16;
+  const int32_t nch = hd.y & 0xffff;
+  const int32_t ng = (nch + kVarChunk - 1) / kVarChunk;
+  const float* part = partial + hd.z;
+  for (int32_t s0 = 0; s0 < ns; s0 += 2) {  // two states at a time
+    const bool pair = s0 + 1 < ns;
+    float t0 = 0.f, t1 = 0.f;
+    for (int32_t j0 = 0; j0 < ng; j0 += 64) {
+      const int32_t k = (j0 + lane) * kVarChunk, k1 = min(nch, k + kVarChunk);
+      float g0 = 0.f, g1 = 0.f;
+      if (ns == 2) {
+        if (k < k1) sum_range2(part, k, k1, g0, g1);
+      } else {
+        for (int32_t i = k; i < k1; ++i) {
+          g0 += part[i * ns + s0];
+          if (pair) g1 += part[i * ns + s0 + 1];
+        }
+      }
+      const int32_t n = min(64, ng - j0);
+      for (int32_t j = 0; j < n; ++j) {
+        t0 += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g0), j));
+        t1 += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(g1), j));
+      }
+    }
+    if (lane == 0) {
+      out[vs0 + s0] = t0 + ev[vs0 + s0];
+      if (pair) out[vs0 + s0 + 1] = t1 + ev[vs0 + s0 + 1];
+    }
   }
 }
 
@@ -2252,21 +2277,6 @@ __device__ __forceinline__ void heavy_chunk_row(const DevGraph& g, int32_t i, co
     }
     partial[slot] = s0;
     partial[slot + 1] = s1;
-  }
-}
-
-// Group sum number gi of a variable with more than kVarChunk chunks.
-__device__ __forceinline__ void heavy_group(const DevGraph& g, int32_t gi, float* partial) {
-  const int32_t h = g.vh_group_h[gi], j = g.vh_group_j[gi];
-  const int32_t v = g.heavy_vars[h];
-  const int32_t ns = g.var_vs0[v + 1] - g.var_vs0[v];
-  const int32_t nch = g.heavy_cptr[h + 1] - g.heavy_cptr[h];
-  const float* part = partial + g.heavy_pofs[h];
-  const int32_t k1 = min(nch, (j + 1) * kVarChunk);
-  for (int32_t s = 0; s < ns; ++s) {
-    float gs = 0.f;
-    for (int32_t k = j * kVarChunk; k < k1; ++k) gs += part[k * ns + s];
-    partial[g.heavy_gpofs[h] + j * ns + s] = gs;
   }
 }
 

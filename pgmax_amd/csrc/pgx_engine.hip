@@ -343,7 +343,7 @@ int pgx_graph_create(const pgx_wiring* wiring, pgx_graph** out) {
   };
   int32_t *var_vs0, *var_eptr, *var_adj_es, *edge_es0, *edge_vs0, *fac_e0, *tables, *heavy;
   int32_t *heavy_cptr, *heavy_pofs, *heavy_chunk_var, *heavy_chunk_k, *edge_var, *perm,
-      *var_adj_ref, *heavy_gpofs, *vh_group_h, *vh_group_j, *heavy_col, *heavy_row,
+      *var_adj_ref, *heavy_groups, *heavy_col, *heavy_row,
       *heavy_stride, *chunk_desc, *chunk_desc_ref, *col_desc, *row_desc, *heavy_desc, *wide_desc;
   Block* blocks;
   Task* tasks;
@@ -355,8 +355,8 @@ int pgx_graph_create(const pgx_wiring* wiring, pgx_graph** out) {
       (rc = up(P.heavy_cptr, &heavy_cptr)) || (rc = up(P.heavy_pofs, &heavy_pofs)) ||
       (rc = up(P.heavy_chunk_var, &heavy_chunk_var)) || (rc = up(P.heavy_chunk_k, &heavy_chunk_k)) ||
       (rc = up(P.edge_var, &edge_var)) || (rc = up(P.perm, &perm)) ||
-      (rc = up(P.var_adj_es_ref, &var_adj_ref)) || (rc = up(P.heavy_gpofs, &heavy_gpofs)) ||
-      (rc = up(P.vh_group_h, &vh_group_h)) || (rc = up(P.vh_group_j, &vh_group_j)) ||
+      (rc = up(P.var_adj_es_ref, &var_adj_ref)) ||
+      (rc = up(P.heavy_groups, &heavy_groups)) ||
       (rc = up(P.heavy_col_chunks, &heavy_col)) || (rc = up(P.heavy_row_chunks, &heavy_row)) ||
       (rc = up(P.heavy_chunk_stride, &heavy_stride)) || (rc = up(P.chunk_desc, &chunk_desc)) ||
       (rc = up(P.chunk_desc_ref, &chunk_desc_ref)) || (rc = up(P.col_desc, &col_desc)) ||
@@ -382,10 +382,8 @@ int pgx_graph_create(const pgx_wiring* wiring, pgx_graph** out) {
   d.heavy_pofs = heavy_pofs;
   d.heavy_chunk_var = heavy_chunk_var;
   d.heavy_chunk_k = heavy_chunk_k;
-  d.heavy_gpofs = heavy_gpofs;
-  d.vh_group_h = vh_group_h;
-  d.vh_group_j = vh_group_j;
-  d.num_vh_groups = int32_t(P.vh_group_h.size());
+  d.heavy_groups = heavy_groups;
+  d.num_heavy_groups = int32_t(P.heavy_groups.size());
   d.heavy_chunk_stride = heavy_stride;
   d.chunk_desc = reinterpret_cast<const int4*>(chunk_desc);
   d.col_desc = reinterpret_cast<const int4*>(col_desc);

@@ -605,24 +605,9 @@ int build_plan(const pgx_wiring& w, Plan* P, std::string* err, int64_t merge_bel
     P->heavy_cptr.push_back(P->heavy_cptr.back() + nch);
     P->heavy_pofs.push_back(P->heavy_pofs.back() + nch * ns);
   }
-  // group sums of variables with more than kVarChunk chunks
-  int64_t gslot = P->heavy_pofs.back();
-  P->heavy_gpofs.assign(P->heavy_vars.size(), -1);
-  for (int32_t h = 0; h < int32_t(P->heavy_vars.size()); ++h) {
-    const int32_t v = P->heavy_vars[h];
-    const int32_t nch = P->heavy_cptr[h + 1] - P->heavy_cptr[h];
-    const int32_t ng = (nch + kVarChunk - 1) / kVarChunk;
-    if (ng <= 1) continue;
-    const int32_t ns = P->var_vs0[v + 1] - P->var_vs0[v];
-    P->heavy_gpofs[h] = int32_t(gslot);
-    for (int32_t j = 0; j < ng; ++j) {
-      P->vh_group_h.push_back(h);
-      P->vh_group_j.push_back(j);
-    }
-    gslot += int64_t(ng) * ns;
-  }
-  PGX_REQUIRE(gslot < (int64_t(1) << 31), PGX_EUNSUP, "too many partial sums");
-  P->partial_size = gslot;
+  for (int32_t h = 0; h < int32_t(P->heavy_vars.size()); ++h)
+    if (P->heavy_cptr[h + 1] - P->heavy_cptr[h] > kVarChunk) P->heavy_groups.push_back(h);
+  P->partial_size = P->heavy_pofs.back();
 
   // Chunk order inside each task: chunk number first, variable second, so
   // neighbouring threads sum the same chunk of neighbouring variables (whose
@@ -694,7 +679,7 @@ int build_plan(const pgx_wiring& w, Plan* P, std::string* err, int64_t merge_bel
       PGX_REQUIRE(nch < (1 << 16), PGX_EUNSUP,
                   "variable " << v << " has more than " << (kVarChunk << 16) << " edges");
       P->heavy_desc.insert(P->heavy_desc.end(),
-                           {P->var_vs0[v], nch | (ns << 16), P->heavy_pofs[h], P->heavy_gpofs[h]});
+                           {P->var_vs0[v], nch | (ns << 16), P->heavy_pofs[h], 0});
     }
   }
 

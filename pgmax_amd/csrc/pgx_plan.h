@@ -108,9 +108,6 @@ struct Plan {
   std::vector<int32_t> var_adj_es_ref;
   std::vector<int32_t> heavy_chunk_var;  // [NHC] heavy-variable index of each chunk
   std::vector<int32_t> heavy_chunk_k;    // [NHC] chunk number within its variable
-  // Variables of more than kVarChunk chunks also sum their chunk sums in
-  // groups of kVarChunk: heavy_gpofs[h] is the first group-sum slot (after
-  // all chunk slots) or -1; (vh_group_h, vh_group_j) enumerate the groups.
   // Chunks split for the per-phase variable kernel: "row" chunks hold a
   // binary variable's edges at evenly spaced positions at most kRowStep apart
   // (one 8-lane group reads them together), "col" chunks the rest (one thread
@@ -124,17 +121,17 @@ struct Plan {
   // row_desc in the order of heavy_col_chunks / heavy_row_chunks.
   std::vector<int32_t> chunk_desc, chunk_desc_ref, col_desc, row_desc;
   // Heavy-variable descriptors, 4 ints each: [first variable state,
-  // chunks | ns << 16, first chunk slot, first group slot or -1].
+  // chunks | ns << 16, first chunk slot, 0].
   std::vector<int32_t> heavy_desc;
   // Variables of more than kThreadStates states and at most kVarChunk edges,
   // 4 ints each: [first variable state, states, first adjacency index, edges].
   std::vector<int32_t> wide_desc;
   std::vector<int32_t> heavy_col_chunks;
   std::vector<int32_t> heavy_row_chunks;
-  std::vector<int32_t> heavy_gpofs;
-  std::vector<int32_t> vh_group_h;
-  std::vector<int32_t> vh_group_j;
-  int64_t partial_size = 0;              // chunk + group slots per batch element
+  // Heavy variables of more than kVarChunk chunks, whose chunk sums are added in
+  // several groups of kVarChunk.
+  std::vector<int32_t> heavy_groups;
+  int64_t partial_size = 0;              // chunk slots per batch element
   // (a task's chunks occupy [heavy_cptr[h0], heavy_cptr[h1]) in chunk-major order)
   std::vector<Block> blocks;
   std::vector<Task> tasks;         // ordered by descending work
