@@ -894,6 +894,12 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
             int64_t(batch) * d.num_es <= (int64_t(1) << 22))
                ? 128
                : 256;
+  // OR / AND graphs gather across their factors' order (an output variable's
+  // AND edge and its far OR edge), so neighbouring workgroups share lines:
+  // untuned, runs of 8 of them go to one XCD (deconvolution images of 40 x 40,
+  // 15 iterations: two 835 -> 793 us, six 1,814 -> 1,664, 24 4,032 -> 3,962;
+  // runs of 64 1,702 and of 256 1,907 for six).
+  if (xcd == 0 && !chosen && (g->kinds_mask & ((1 << kOr) | (1 << kAnd)))) xcd = 8;
   r.xcd = int32_t(std::max<int64_t>(0, std::min<int64_t>(xcd, 1024)));
   // k_bipartite numbers (tile, batch element) pairs in one grid dimension
   const int64_t bip_units = int64_t((d.bip_na + d.bip_unary + kBipRows - 1) / kBipRows) *
