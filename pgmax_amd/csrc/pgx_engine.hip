@@ -462,6 +462,7 @@ int pgx_graph_create(const pgx_wiring* wiring, pgx_graph** out) {
     }
   }
   d.fusable = (P.pairwise_only && P.max_degree <= kFuseMaxDeg) ? 1 : 0;
+  g->wide_plan = P.wide_only && !P.edge_pos4.empty() ? 1 : 0;
   g->packed_plan = P.packable ? 1 : 0;
   g->even2_plan = P.even2;
   g->fusable_plan = d.fusable;
@@ -934,6 +935,7 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
   // or kFusedMaxStates edge states its two-kernel iteration is faster.
   g->dev.fusable =
       (g->fusable_plan && fuse && (fuse == 2 || chosen || small_run || mode != 2)) ? 1 : 0;
+  g->dev.wide_fused = (g->wide_plan && fuse && (fuse == 2 || chosen || small_run)) ? 1 : 0;
   const bool t0 = (temperature == 0.f);
   KernelClock clk;
   clk.on = prof == 2;
@@ -1207,7 +1209,7 @@ int pgx_autotune(pgx_graph* g, const float* lp, int64_t lp_stride, const float* 
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int32_t n_it = std::max(probe_iters, 2);
   std::vector<RunCfg> cands;
-  const bool can_fuse = g->fusable_plan || g->bip_plan;
+  const bool can_fuse = g->fusable_plan || g->bip_plan || g->wide_plan;
   const int64_t fuse_opts[2] = {can_fuse ? 1 : 0, 0};
   const int nf = can_fuse ? 2 : 1;
   for (int fi = 0; fi < nf; ++fi)

@@ -322,6 +322,7 @@ struct pgx_graph {
   int32_t kinds_mask = 0;
   int32_t num_tiles = 0;
   int32_t fusable_plan = 0;
+  int32_t wide_plan = 0;    // wide pairwise factors may form the sums (Plan::wide_only)
   int32_t bip_plan = 0;     // complete bipartite binary graph (k_bipartite applies)
   pgx::DevPatches patches;  // count 0: none
   int32_t packed_plan = 0;  // 2x2 factors only, binary variables of <= 4 edges (Plan::packable)

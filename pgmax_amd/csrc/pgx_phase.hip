@@ -195,8 +195,8 @@ __device__ __forceinline__ void fac_phase_body(const DevGraph& g, const Tile* ti
       const int32_t i = tile.i0 + w * fw + fl;
       // per factor: its edge states, then its summaries
       float* xs = wl[w] + fl * (blk.esf + blk.s0 * (blk.s1 | 1));
-      pair_wide<kT0>(g, blk, i, fl < fw && i < tile.i1, lane - fl * blk.esf, io, t, dl, xs,
-                     xs + blk.esf);
+      pair_wide<kT0>(g, blk, i, fl < fw && i < tile.i1, lane - fl * blk.esf, io,
+                     g.wide_fused ? r.ev + b * r.ev_stride : nullptr, t, dl, xs, xs + blk.esf);
       block_delta_store<kPhaseThreads>(dl, delta_dst<kConv>(g, r, blk, b, it));
       return;
     }
@@ -676,7 +676,7 @@ static int launch_phased_t(pgx_graph* g, const RunBufs& r, int32_t batch, hipStr
                            : with_shared_tables(d, nullptr, 0, r, batch, s);
   for (int32_t it = 0; it < rr.n_it; ++it) {
     const float* mo = ((rr.n_it - it) & 1) ? rr.y : rr.x;
-    if (d.num_vars > 0)
+    if (d.num_vars > 0 && !d.wide_fused)
       launch_var_phase(d, mo, d.num_es, rr.ev, rr.ev_stride, rr.vsum, rr.partial, batch, s, &clk,
                        rr.xcd);
     launch_fac_kinds<kT0, kConv>(g, M, rr, batch, it, s, clk, lanes);

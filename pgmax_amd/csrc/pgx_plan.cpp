@@ -507,7 +507,9 @@ int build_plan(const pgx_wiring& w, Plan* P, std::string* err, int64_t merge_bel
   for (int32_t v = 0; v < NV; ++v)
     P->max_degree = std::max(P->max_degree, P->var_eptr[v + 1] - P->var_eptr[v]);
   P->pairwise_only = !P->blocks.empty();
+  P->wide_only = !P->blocks.empty() && P->max_degree <= 4;
   for (Block& b : P->blocks) {
+    if (b.kind != kEnumGeneral || !(b.pad[0] & 32)) P->wide_only = false;
     if (b.kind != kEnumBin2 && b.kind != kEnumPair) P->pairwise_only = false;
     if (b.kind == kEnumBin2 && b.c0 % 4 == 0) b.pad[0] |= 1;
     // general Enum factors with a wavefront's worth of rows and tables that
@@ -561,7 +563,7 @@ int build_plan(const pgx_wiring& w, Plan* P, std::string* err, int64_t merge_bel
       }
       for (int32_t k = 0; k < deg; ++k) P->var_pos4[size_t(v) * 4 + k] = P->var_adj_es[p0 + k];
     }
-    if (P->pairwise_only && int64_t(E) * 16 <= kEdgePos4MaxBytes) {
+    if ((P->pairwise_only || P->wide_only) && int64_t(E) * 16 <= kEdgePos4MaxBytes) {
       P->edge_pos4.resize(size_t(E) * 4);
       for (int32_t e = 0; e < E; ++e)
         for (int k = 0; k < 4; ++k)

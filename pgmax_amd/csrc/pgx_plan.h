@@ -139,6 +139,9 @@ struct Plan {
   std::vector<int32_t> edge_var;   // [E] variable of each edge
   int32_t max_degree = 0;          // most edges on one variable
   bool pairwise_only = false;      // every factor is a full-table pairwise Enum factor
+  // Every factor a full pairwise table run with one lane per edge state (Block
+  // bit 5) and every variable of at most 4 edges.
+  bool wide_only = false;
   // Variables of at most 4 edges: their edges' engine positions in edge
   // order, 4 ints per variable (-1 past the degree; -2 in slot 0 for more
   // than 4 edges), so a variable sum needs one index load. edge_pos4 holds
