@@ -1239,7 +1239,9 @@ int pgx_autotune(pgx_graph* g, const float* lp, int64_t lp_stride, const float* 
         for (int64_t x : {4, 16}) cands.push_back(RunCfg{2, 0, 1, 3, 256, 1, x});
       }
     }
-  if (converge)  // per-phase launches that skip the tasks that are done
+  // per-phase launches that skip the tasks that are done, where untuned runs
+  // may take them
+  if (converge && converge_shape(g, batch, n_it, temperature == 0.f).first == 2)
     for (int fi = g->fusable_plan ? 0 : 1; fi < 2; ++fi)
       for (int64_t t : {64, 128, 256}) cands.push_back(RunCfg{2, 0, fi == 0 ? 1 : 0, 3, t});
   if (!converge && g->patches.count > 0) cands.push_back(RunCfg{4, 0, 1, 3, 256});
