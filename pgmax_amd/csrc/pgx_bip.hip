@@ -50,6 +50,8 @@ __global__ void __launch_bounds__(kThreads)
   constexpr int kStep = kThreads / kCols;  // rows one pass of the workgroup covers
   constexpr int kPer = kBipRows / kStep;   // rows per thread
   static_assert(kPer * kStep == kBipRows, "rows split evenly");
+  constexpr int kColSum = kCols < 64 ? 64 : kCols;  // first thread of the columns' chunk sums
+  static_assert(kThreads >= kColSum + kCols, "a thread per column chunk");
   __shared__ float2 srow[kBipRows][kCols + 1];  // new messages of the rows' edges (padded)
   __shared__ float2 scol[kBipRows][kCols];      // new messages of the columns' edges
   __shared__ float2 vrow[kBipRows];             // variable sums of the tile's rows
@@ -251,8 +253,8 @@ __global__ void __launch_bounds__(kThreads)
       }
       st2(pout + g.bip_row[a0 + ra - U].y + 2 * ((c0 + cb) / kVarChunk), s0, s1);
     }
-  } else if (tid < 2 * kCols && tid - kCols < ncl && c0 + (tid - kCols) >= U) {
-    const int32_t c = tid - kCols;  // column chunks: thread = column
+  } else if (tid >= kColSum && tid - kColSum < ncl && c0 + (tid - kColSum) >= U) {
+    const int32_t c = tid - kColSum;  // column chunks: thread = column, in other wavefronts
     float s0 = 0.f, s1 = 0.f;
     if (nr == kBipRows) {
       float2 m[kBipRows];
@@ -299,6 +301,8 @@ void launch_bipartite(const DevGraph& d, const RunBufs& r, const float* msg_in, 
   if (cols != 32 && cols != 64 && cols != 128) cols = 32;
   if (cols == 32 && threads == 128)
     launch_bipartite_t<kT0, 32, 128>(d, r, msg_in, msg_out, pin, pout, it, batch, s);
+  else if (cols == 32 && threads == 512)
+    launch_bipartite_t<kT0, 32, 512>(d, r, msg_in, msg_out, pin, pout, it, batch, s);
   else if (cols == 32)
     launch_bipartite_t<kT0, 32, 256>(d, r, msg_in, msg_out, pin, pout, it, batch, s);
   else if (cols == 128)

@@ -928,7 +928,11 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
     const int64_t per_task = (int64_t(d.num_es) + d.num_vs) / std::max<int64_t>(d.num_tasks, 1);
     mode = (wgs >= 256 && per_task <= 4096) ? 1 : 2;
   }
-  if (bs == 0) bs = 256;
+  // (complete bipartite graphs of at most two tiles per CU: two factors a thread
+  // in place of four. us an iteration: one RBM 500 x 100 with biases, T = 0, 9.5
+  // -> 7.9; 800 x 200, T = 1, 14.0 -> 10.9; 8 of 500 x 100 11.1 -> 10.7, 16 of
+  // them 15.1 and 15.9)
+  if (bs == 0) bs = (g->dev.bip && mode == 2 && tile == 256 && bip_units <= 512) ? 512 : 256;
   // Untuned, the per-phase shape recomputes variable sums on the factor side
   // (one launch per iteration, every variable's messages re-read per factor)
   // only for small runs, where the launch count dominates; past kFusedMaxBin2
