@@ -280,3 +280,36 @@ def test_logical_blocks_match_oracle(gpu, kind, logical, temperature):
     np.testing.assert_array_equal(_np(d), ref_d)
   np.testing.assert_array_equal(_np(bp.context.get_flat_beliefs(out)),
                                 lbp.get_flat_beliefs(graph, ref, ev))
+
+
+@pytest.mark.parametrize("sizes", [(2,), (1, 2, 8), (9, 16), (7, 17, 40)])
+def test_map_and_marginals_at_register_sizes(gpu, sizes):
+  """Variables of states that stay in registers and that do not, mixed in a
+  graph, with ties, infinite and NaN beliefs: the oracle's first maximal state
+  and softmax."""
+  import torch
+  groups = [vgroup.NDVarArray(num_states=s, shape=(70,)) for s in sizes]
+  fg = fgraph.FactorGraph(variable_groups=groups)
+  for g in groups:
+    n = g.num_states.reshape(-1)[0]
+    fg.add_factors(fgroup.EnumFactorGroup(variables_for_factors=[[g[i]] for i in range(70)],
+                                          factor_configs=np.arange(n)[:, None]))
+  bp = infer.BP(fg.bp_state, temperature=1.0)
+  eng = bp.context.engine
+  rng = np.random.default_rng(3)
+  ev = rng.integers(-3, 3, size=eng.graph.num_vs).astype(np.float32)  # (ties)
+  ev[5] = np.nan
+  ev[-3] = -np.inf
+  ev[-1] = np.inf
+  ft = np.zeros(eng.graph.num_es, np.float32)
+  bel, dec, marg = (_np(x) for x in eng.beliefs_decode(ev, ft))
+  np.testing.assert_array_equal(bel, ev)
+  at = 0
+  for i, s in enumerate(np.repeat(sizes, 70)):
+    x = bel[at:at + s]
+    assert dec[i] == np.argmax(x), (i, x)
+    if np.isfinite(x).all():
+      e = np.exp(x.astype(np.float64) - x.max())
+      np.testing.assert_allclose(marg[at:at + s], e / e.sum(), rtol=1e-6)  # some ulp of exp
+    at += s
+  torch.cuda.synchronize()
