@@ -68,11 +68,11 @@ def rocprof_key(kernel, temperature, lanes=False):
   lanes: square pairwise tables ran on lane groups (k_pair_lanes)."""
   t0 = "true" if temperature == 0.0 else "false"
   if kernel == "fac_phase_enum_pair" and lanes:
-    return f"k_pair_lanes<{t0}>"
+    return f"k_pair_lanes<{t0}, "
   if kernel == "fac_fused" and lanes:
-    return f"k_pair_lanes_fused<{t0}>"
+    return f"k_pair_lanes_fused<{t0}, "
   if kernel in FAC_KINDS:
-    return f"k_fac_phase<{t0}, {FAC_KINDS[kernel]}>"
+    return f"k_fac_phase<{t0}, {FAC_KINDS[kernel]}, "
   return {"bipartite": f"k_bipartite<{t0}, ", "var_phase": "k_var_phase",
           "fac_fused": f"k_fac_fused<{t0}, ", "task_loop": "k_task_loop<",
           "vjp_pair_bwd": "k_pair_bwd<", "vjp_pair_fwd": "k_pair_fwd<",
