@@ -1756,8 +1756,6 @@ __device__ void pool_factor(const DevGraph& g, int32_t f, const IO& io, float t,
 // Sets of block kinds a kernel is compiled for (bit k = BlockKind k). A
 // kernel only holds the code of its kinds, which keeps the lean pairwise
 // paths free of the register pressure of the general ones.
-constexpr int kKindsBin2 = 1 << kEnumBin2;
-constexpr int kKindsPairwise = (1 << kEnumBin2) | (1 << kEnumPair);
 constexpr int kKindsAll = 0x3f;
 
 // Dispatches factor i of block b (b.kind must be in KINDS).

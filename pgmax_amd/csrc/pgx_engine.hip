@@ -699,39 +699,6 @@ static inline bool aligned(const void* p, uintptr_t a) {
   return (reinterpret_cast<uintptr_t>(p) & (a - 1)) == 0;
 }
 
-// Untuned shape of a convergence run: {mode, threads per task-loop workgroup}.
-// The task loop (1) stops each task's workgroup at its convergence, but an
-// iteration takes one CU the whole task: about 0.65 ns per edge or variable
-// state of 2x2 graphs at T > 0, 1.3 ns with larger tables, under half of it
-// at T = 0 (us_iter: the largest task, or the CUs' share of all tasks). The
-// per-phase launches (2) spread every iteration over the chip, but all n_it
-// of them are launched, 2.7 us each also after the last task is done. They
-// are taken where an iteration of the task loop is long (20 us) and the idle
-// launches cost at most about 20 of them. Measured, 300 iterations allowed:
-// 100 x 100 torus 46.5 ms (task loop, 256 threads) -> 2.0 ms; 300 Potts grids
-// 40 x 40 x 8, done after 26 on average, 10.3 -> 4.6; 10 x 10 torus, done
-// after 69, stays in the task loop (0.24 ms against 1.3). Workgroups of the
-// task loop: 30 x 30 torus 1,416 us with 256 threads, 634 with 1,024; 16 x 16
-// Potts grid of 8 states 328 with 256, 281 with 512, 323 with 1,024; 4,096
-// 10 x 10 tori 1.8 ms with 256, 2.8 with 512.
-static std::pair<int64_t, int64_t> converge_shape(const pgx_graph* g, int32_t batch, int32_t n_it,
-                                           bool t0) {
-  const Plan& P = g->plan;
-  const Task& big = P.tasks[0];  // ordered by descending work
-  int64_t total = 0, factors = 0;
-  for (const Task& t : P.tasks) total += t.work;
-  for (int32_t bi = big.b0; bi < big.b1; ++bi) factors += P.blocks[bi].count;
-  const bool bin2 = g->kinds_mask == kKindsBin2;
-  const double ns = (bin2 ? 0.65 : 1.3) * (t0 ? 0.45 : 1.0);
-  const double us_iter =
-      1e-3 * ns * double(std::max(big.work, total * batch / 256));
-  if (us_iter >= 20.0 && 20.0 * us_iter >= 2.7 * n_it) return {2, 0};
-  const int64_t wgs = int64_t(P.tasks.size()) * batch;
-  if (bin2 && factors >= 512) return {1, wgs <= 512 ? 1024 : 512};
-  if ((g->kinds_mask & ~kKindsPairwise) == 0 && factors >= 256) return {1, 512};
-  return {1, 256};
-}
-
 // Untuned runs take k_patch where the graph is small enough: whole components
 // always (16 x 16 tori, us an iteration at T = 1 against the task loop's 512
 // threads: one 1.5 and 3.9, 256 of them 1.7 and 4.1, 1,000 6.1 and 8.2),
@@ -965,7 +932,8 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
   g->dev.lp_al4 = ((vec & 2) && lp_stride % 4 == 0 && aligned(lp, 16)) ? ((vec & 4) ? 2 : 1) : 0;
   g->dev.lp_nt = (vec & 4) ? 1 : 0;
   if (converge && mode == 0) {
-    const auto shape = converge_shape(g, batch, n_it, temperature == 0.f);
+    const auto shape =
+        converge_shape(g->plan, g->kinds_mask, batch, n_it, temperature == 0.f);
     mode = shape.first;
     if (bs == 0) bs = shape.second;
   }
@@ -1297,7 +1265,8 @@ int pgx_autotune(pgx_graph* g, const float* lp, int64_t lp_stride, const float* 
     }
   // per-phase launches that skip the tasks that are done, where untuned runs
   // may take them
-  if (converge && converge_shape(g, batch, n_it, temperature == 0.f).first == 2)
+  if (converge &&
+      converge_shape(g->plan, g->kinds_mask, batch, n_it, temperature == 0.f).first == 2)
     for (int fi = g->fusable_plan ? 0 : 1; fi < 2; ++fi)
       for (int64_t t : {64, 128, 256}) cands.push_back(RunCfg{2, 0, fi == 0 ? 1 : 0, 3, t});
   if (!converge && g->patches.count > 0) cands.push_back(RunCfg{4, 0, 1, 3, 256});

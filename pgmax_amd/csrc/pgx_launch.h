@@ -19,6 +19,7 @@
 #include "pgx_device.h"
 #include "pgx_internal.h"
 #include "pgx_plan.h"
+#include "pgx_shape.h"
 
 namespace pgx {
 

@@ -25,6 +25,10 @@ enum BlockKind : int32_t {
   kPool = 5,
 };
 
+// Sets of block kinds (bit k = BlockKind k).
+constexpr int kKindsBin2 = 1 << kEnumBin2;
+constexpr int kKindsPairwise = (1 << kEnumBin2) | (1 << kEnumPair);
+
 struct Block {
   int32_t kind;
   int32_t task;    // index in Plan::tasks

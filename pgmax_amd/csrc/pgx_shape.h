@@ -1,0 +1,33 @@
+// Host rules that choose how a run is executed: plain functions of the plan
+// and the call's sizes, so they can be tested without a GPU.
+#ifndef PGX_SHAPE_H_
+#define PGX_SHAPE_H_
+
+#include <utility>
+
+#include "pgx_plan.h"
+
+namespace pgx {
+
+// Untuned shape of a convergence run: {mode, threads per task-loop workgroup}.
+// The task loop (1) stops each task's workgroup at its convergence, but an
+// iteration takes one CU the whole task: about 0.65 ns per edge or variable
+// state of 2x2 graphs at T > 0, 1.3 ns with larger tables, under half of it
+// at T = 0 (us_iter: the largest task, or the CUs' share of all tasks). The
+// per-phase launches (2) spread every iteration over the chip, but all n_it
+// of them are launched, 2.7 us each also after the last task is done. They
+// are taken where an iteration of the task loop is long (20 us) and the idle
+// launches cost at most about 20 of them. Measured, 300 iterations allowed:
+// 100 x 100 torus 46.5 ms (task loop, 256 threads) -> 2.0 ms; 300 Potts grids
+// 40 x 40 x 8, done after 26 on average, 10.3 -> 4.6; 10 x 10 torus, done
+// after 69, stays in the task loop (0.24 ms against 1.3). Workgroups of the
+// task loop: 30 x 30 torus 1,416 us with 256 threads, 634 with 1,024; 16 x 16
+// Potts grid of 8 states 328 with 256, 281 with 512, 323 with 1,024; 4,096
+// 10 x 10 tori 1.8 ms with 256, 2.8 with 512.
+// A graph without factors has no tasks, and its runs launch no iterations.
+std::pair<int64_t, int64_t> converge_shape(const Plan& plan, int32_t kinds_mask, int32_t batch,
+                                           int32_t n_it, bool t0);
+
+}  // namespace pgx
+
+#endif  // PGX_SHAPE_H_

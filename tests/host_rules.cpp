@@ -1,0 +1,37 @@
+// Test doors into the library's host rules (pgx_plan.cpp, pgx_shape.cpp), built
+// with the host compiler by test_host_rules.py: no GPU, no HIP.
+
+#include "../pgmax_amd/csrc/pgx_plan.h"
+#include "../pgmax_amd/csrc/pgx_shape.h"
+
+using namespace pgx;
+
+namespace {
+
+int plan_of(const pgx_wiring* w, Plan* P, int32_t* kinds) {
+  std::string err;
+  const int rc = build_plan(*w, P, &err, 4096, true);
+  *kinds = 0;
+  for (const Block& b : P->blocks) *kinds |= 1 << b.kind;
+  return rc;
+}
+
+}  // namespace
+
+extern "C" {
+
+// Untuned shape of a convergence run: [tasks, mode, threads].
+int rules_converge_shape(const pgx_wiring* w, int32_t batch, int32_t n_it, int32_t t0,
+                         int64_t* out) {
+  Plan P;
+  int32_t kinds;
+  const int rc = plan_of(w, &P, &kinds);
+  if (rc) return rc;
+  const auto shape = converge_shape(P, kinds, batch, n_it, t0 != 0);
+  out[0] = int64_t(P.tasks.size());
+  out[1] = shape.first;
+  out[2] = shape.second;
+  return 0;
+}
+
+}  // extern "C"

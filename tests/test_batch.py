@@ -221,6 +221,18 @@ def test_autotune_keeps_results(gpu):
   assert cfg_c["mode"] == 1
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("converge", [False, True])
+def test_autotune_of_a_graph_without_factors(gpu, converge):
+  """Variables and no factors: every shape's run is empty, and one is chosen."""
+  bb = batch.BatchedBP([batch.grid_wiring(1, 1, 3, full_tables=True)] * 2, temperature=1.0)
+  assert bb.graph.num_tasks == 0 and bb.graph.num_es == 0
+  ev = np.arange(6, dtype=np.float32)
+  cfg = bb.autotune(np.zeros(0, np.float32), None, ev, converge=converge, probe_iters=3)
+  assert cfg["mode"] in (1, 2)
+  np.testing.assert_array_equal(bb.beliefs(ev, np.zeros(0, np.float32)).cpu().numpy(), ev)
+
+
 def test_deconvolution_wiring_matches_factor_graph():
   """The direct builder equals FactorGraph + AND/OR factor groups built as in
   the reference's deconvolution notebook (cells 12-14), on a small instance."""

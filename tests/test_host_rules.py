@@ -1,0 +1,47 @@
+"""The library's host rules (plans and execution shapes) as plain functions,
+built with the host compiler: no GPU needed."""
+
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+from pgmax_amd import batch
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CSRC = os.path.join(HERE, "..", "pgmax_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+  lib = str(tmp_path_factory.mktemp("rules") / "rules.so")
+  subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared",
+                  os.path.join(HERE, "host_rules.cpp"), os.path.join(CSRC, "pgx_plan.cpp"),
+                  os.path.join(CSRC, "pgx_shape.cpp"), "-o", lib], check=True)
+  return ctypes.CDLL(lib)
+
+
+def _converge_shape(rules, flat, n_it, batch_size=1, t0=False):
+  w = flat.to_engine_wiring()
+  out = (ctypes.c_int64 * 3)()
+  assert rules.rules_converge_shape(ctypes.byref(w.struct), batch_size, n_it, int(t0), out) == 0
+  return tuple(out)
+
+
+def test_convergence_shape_of_a_graph_without_factors(rules):
+  """No factors, no tasks: the rule answers (any shape, nothing is launched)."""
+  lone = batch.grid_wiring(1, 1, 3, full_tables=True)
+  assert lone.num_edge_states == 0 and lone.num_var_states == 3
+  assert _converge_shape(rules, lone, 10) == (0, 1, 256)
+
+
+@pytest.mark.parametrize("side,n_it,want", [
+    (10, 300, (1, 256)),    # iterations of microseconds: task loop
+    (30, 300, (1, 1024)),
+    (100, 300, (2, 0)),     # long iterations, few idle launches
+    (100, 5000, (1, 1024)),  # too many launches that might be idle
+])
+def test_convergence_shape_by_iterations_allowed(rules, side, n_it, want):
+  torus = batch.grid_wiring(side, side, 2, torus=True, full_tables=True)
+  assert _converge_shape(rules, torus, n_it)[1:] == want
