@@ -840,7 +840,8 @@ void split_compact(const FactorNeighbours& nb, std::vector<int32_t> fs, int32_t 
 
 Patches build_patches(const Plan& P) {
   const int32_t F = P.num_factors;
-  if (F == 0 || P.max_degree > 4 || P.num_edges != 2 * F) return {};
+  if (F == 0 || P.max_degree > 4 || P.num_edges != 2 * F || !patch_edges_fit(P.num_edges))
+    return {};
   std::vector<int32_t> lp0(static_cast<size_t>(F));
   int32_t largest = 0;  // factors of a task
   for (const Task& t : P.tasks) {

@@ -210,6 +210,11 @@ constexpr int32_t kPatchOwn = 80;            // own factors aimed at with rings
 constexpr int32_t kPatchMaxFactors = 1 << 15;  // of a graph with rings
 constexpr int32_t kPatchRingShift = 28;
 constexpr int32_t kPatchEdgeMask = (1 << kPatchRingShift) - 1;
+// A patch's threads hold their edge in the bits below the ring: the edges of a
+// graph that has patches.
+constexpr bool patch_edges_fit(int64_t num_edges) {
+  return num_edges <= int64_t(kPatchEdgeMask) + 1;
+}
 // Empty when the graph is of another kind or too large.
 Patches build_patches(const Plan& plan);
 

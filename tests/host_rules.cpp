@@ -34,4 +34,26 @@ int rules_converge_shape(const pgx_wiring* w, int32_t batch, int32_t n_it, int32
   return 0;
 }
 
+// Patches of a graph: [patches, depth], or of one that only states its size
+// (w null): num_edges / 2 factors, and a task with none of them.
+int rules_patches(const pgx_wiring* w, int64_t num_edges, int64_t* out) {
+  Plan P;
+  int32_t kinds;
+  if (w) {
+    const int rc = plan_of(w, &P, &kinds);
+    if (rc) return rc;
+  } else {
+    P.num_edges = int32_t(num_edges);
+    P.num_factors = int32_t(num_edges / 2);
+    P.max_degree = 4;
+    P.tasks.push_back(Task{});
+  }
+  const Patches p = build_patches(P);
+  out[0] = p.count;
+  out[1] = p.depth;
+  return 0;
+}
+
+int rules_patch_edges_fit(int64_t num_edges) { return patch_edges_fit(num_edges) ? 1 : 0; }
+
 }  // extern "C"

@@ -45,3 +45,19 @@ def test_convergence_shape_of_a_graph_without_factors(rules):
 def test_convergence_shape_by_iterations_allowed(rules, side, n_it, want):
   torus = batch.grid_wiring(side, side, 2, torus=True, full_tables=True)
   assert _converge_shape(rules, torus, n_it)[1:] == want
+
+
+def test_patches_take_edge_numbers_of_28_bits(rules):
+  """A patch's threads hold their edge in 28 bits under its ring: graphs with
+  more edges have no patches, whatever their components' size."""
+  out = (ctypes.c_int64 * 2)()
+  for flat in (batch.grid_wiring(16, 16, 2, torus=True, full_tables=True),
+               batch.grid_wiring(17, 16, 2, torus=True, full_tables=True)):
+    w = flat.to_engine_wiring()
+    assert rules.rules_patches(ctypes.byref(w.struct), ctypes.c_int64(0), out) == 0
+    assert out[0] > 0
+  fit = lambda n: rules.rules_patch_edges_fit(ctypes.c_int64(n))
+  assert fit(0) and fit(2) and fit(2**28 - 2) and fit(2**28)
+  assert not fit(2**28 + 1) and not fit(2**28 + 2) and not fit(2**31 - 2)
+  assert rules.rules_patches(None, ctypes.c_int64(2**28 + 2), out) == 0
+  assert out[0] == 0
