@@ -153,7 +153,9 @@ int pgx_run_converge(pgx_graph* graph,
  * inputs for probe_iters iterations, and makes the fastest the graph's
  * shape for later pgx_run (converge = 0) or pgx_run_converge (converge = 1)
  * calls with the same batch size and temperature class (0 or > 0), as long
- * as the "mode", "block" and "tile" options are 0. Per-phase shapes are
+ * as the "mode", "block" and "tile" options are 0. Of a convergence run it
+ * also keeps the fastest task-loop shape, which runs take whose max_iters
+ * would leave too many per-phase launches idle after the last task stops. Per-phase shapes are
  * tried with 64, 128 and 256 factors per workgroup, the complete bipartite
  * iteration with tiles of 32 rows x 32, 64 or 128 columns and 256 or 512
  * threads, and per-phase runs with square pairwise tables both on S lanes

@@ -893,13 +893,15 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
   } else if (mode == 0 && bs == 0 && tile == 0) {
     auto it = g->tuned.find(std::make_tuple(batch, temperature == 0.f ? 1 : 0, converge ? 1 : 0));
     if (it != g->tuned.end()) {
-      mode = it->second.mode;
-      bs = it->second.bs;
-      fuse = it->second.fuse;
-      vec = it->second.vec;
-      tile = it->second.tile;
-      lanes = it->second.lanes;
-      xcd = it->second.xcd;
+      const RunCfg& c = tuned_shape(it->second, converge, g->plan, g->kinds_mask, batch, n_it,
+                                    temperature == 0.f);
+      mode = c.mode;
+      bs = c.bs;
+      fuse = c.fuse;
+      vec = c.vec;
+      tile = c.tile;
+      lanes = c.lanes;
+      xcd = c.xcd;
       chosen = true;
     }
   }
@@ -1264,9 +1266,8 @@ int pgx_autotune(pgx_graph* g, const float* lp, int64_t lp_stride, const float* 
       }
     }
   // per-phase launches that skip the tasks that are done, where untuned runs
-  // may take them
-  if (converge &&
-      converge_shape(g->plan, g->kinds_mask, batch, n_it, temperature == 0.f).first == 2)
+  // of few enough iterations take them (tuned_shape looks at each run's count)
+  if (converge && converge_shape(g->plan, g->kinds_mask, batch, 1, temperature == 0.f).first == 2)
     for (int fi = g->fusable_plan ? 0 : 1; fi < 2; ++fi)
       for (int64_t t : {64, 128, 256}) cands.push_back(RunCfg{2, 0, fi == 0 ? 1 : 0, 3, t});
   if (!converge && g->patches.count > 0) cands.push_back(RunCfg{4, 0, 1, 3, 256});
@@ -1290,11 +1291,11 @@ int pgx_autotune(pgx_graph* g, const float* lp, int64_t lp_stride, const float* 
   int rc = PGX_OK;
   if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
     rc = set_error(PGX_EHIP, "pgx_autotune: hipEventCreate failed");
-  RunCfg best;
-  float best_ms = 3.4e38f;
+  Tuned tuned;
+  float best_ms = 3.4e38f, loop_ms = 3.4e38f;
   for (const RunCfg& c : cands) {
     if (rc) break;
-    float ms = 3.4e38f;
+    float ms = 3.4e38f, first_ms = 3.4e38f;
     for (int rep = 0; rep < 3 && !rc; ++rep) {  // first repetition warms up
       (void)hipEventRecord(e0, s);
       rc = converge ? run_impl(g, lp, lp_stride, ev, ev_stride, ftov_in, ftov_in_stride, out,
@@ -1312,12 +1313,19 @@ int pgx_autotune(pgx_graph* g, const float* lp, int64_t lp_stride, const float* 
       float t = 0.f;
       (void)hipEventElapsedTime(&t, e0, e1);
       if (rep > 0) ms = std::min(ms, t);
+      else first_ms = t;
       // a shape whose first run takes 4x the best shape's time cannot win
       if (rep == 0 && best_ms < 3.4e38f && t > 4.f * best_ms) break;
     }
     if (!rc && ms < best_ms) {
       best_ms = ms;
-      best = c;
+      tuned.best = c;
+    }
+    // (a loop shape cut short at its first repetition is kept by that time)
+    const float lm = ms < 3.4e38f ? ms : first_ms;
+    if (!rc && c.mode == 1 && lm < loop_ms) {
+      loop_ms = lm;
+      tuned.task_loop = c;
     }
   }
   (void)hipEventDestroy(e0);
@@ -1326,8 +1334,9 @@ int pgx_autotune(pgx_graph* g, const float* lp, int64_t lp_stride, const float* 
   (void)hipFree(dl);
   (void)hipFree(it_done);
   if (rc) return rc;
-  g->tuned[std::make_tuple(batch, temperature == 0.f ? 1 : 0, converge ? 1 : 0)] = best;
+  g->tuned[std::make_tuple(batch, temperature == 0.f ? 1 : 0, converge ? 1 : 0)] = tuned;
   if (chosen) {
+    const RunCfg& best = tuned.best;
     chosen[0] = best.mode;
     chosen[1] = best.bs;
     chosen[2] = best.fuse;

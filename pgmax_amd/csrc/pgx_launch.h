@@ -263,12 +263,6 @@ struct DevPatches {
   const int32_t* extra = nullptr;
 };
 
-// Execution shape of one run: mode 1 task loop / 2 phased, workgroup size of
-// the task loop, factor-side variable sums, vector accesses.
-struct RunCfg {
-  int64_t mode = 0, bs = 0, fuse = 1, vec = 3, tile = 256, lanes = 1, xcd = 0;
-};
-
 // Tile groups: the six block kinds, then (per-phase tile sets only) square
 // pairwise Enum blocks of 3..8 states, once as lane-group tiles
 // (k_pair_lanes) and once one factor per thread (k_fac_phase); a run
@@ -312,7 +306,7 @@ struct pgx_graph {
   // otherwise), with kLaneFusedPasses passes per wavefront (lane_set)
   pgx::TileSet lsets[pgx::kLaneSets];
   // shapes chosen by pgx_autotune, keyed by (batch, temperature == 0, converge)
-  std::map<std::tuple<int32_t, int, int>, pgx::RunCfg> tuned;
+  std::map<std::tuple<int32_t, int, int>, pgx::Tuned> tuned;
   // runs captured as HIP graphs (option "graph"), keyed by every launch argument
   std::map<std::vector<int64_t>, hipGraphExec_t> graphs;
   std::vector<std::vector<int64_t>> graph_order;  // insertion order, for eviction

@@ -24,4 +24,11 @@ std::pair<int64_t, int64_t> converge_shape(const Plan& P, int32_t kinds_mask, in
   return {1, 256};
 }
 
+const RunCfg& tuned_shape(const Tuned& tuned, bool converge, const Plan& plan, int32_t kinds_mask,
+                          int32_t batch, int32_t n_it, bool t0) {
+  const bool other = converge && tuned.best.mode != 1 &&
+                     converge_shape(plan, kinds_mask, batch, n_it, t0).first != 2;
+  return other ? tuned.task_loop : tuned.best;
+}
+
 }  // namespace pgx

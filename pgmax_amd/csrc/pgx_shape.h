@@ -9,6 +9,12 @@
 
 namespace pgx {
 
+// Execution shape of one run: mode 1 task loop / 2 phased, workgroup size of
+// the task loop, factor-side variable sums, vector accesses.
+struct RunCfg {
+  int64_t mode = 0, bs = 0, fuse = 1, vec = 3, tile = 256, lanes = 1, xcd = 0;
+};
+
 // Untuned shape of a convergence run: {mode, threads per task-loop workgroup}.
 // The task loop (1) stops each task's workgroup at its convergence, but an
 // iteration takes one CU the whole task: about 0.65 ns per edge or variable
@@ -27,6 +33,19 @@ namespace pgx {
 // A graph without factors has no tasks, and its runs launch no iterations.
 std::pair<int64_t, int64_t> converge_shape(const Plan& plan, int32_t kinds_mask, int32_t batch,
                                            int32_t n_it, bool t0);
+
+// The autotuner's choice for a batch size and temperature class. Convergence
+// runs also keep their fastest task-loop shape.
+struct Tuned {
+  RunCfg best, task_loop;
+};
+// The shape a tuned run of at most n_it iterations takes. Probes are short and
+// no task finishes in them, so they do not show what per-phase launches that
+// outlast every task cost: a convergence run takes them only where
+// converge_shape lets an untuned run of n_it iterations take them, and the
+// task loop elsewhere.
+const RunCfg& tuned_shape(const Tuned& tuned, bool converge, const Plan& plan, int32_t kinds_mask,
+                          int32_t batch, int32_t n_it, bool t0);
 
 }  // namespace pgx
 

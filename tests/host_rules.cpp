@@ -34,6 +34,18 @@ int rules_converge_shape(const pgx_wiring* w, int32_t batch, int32_t n_it, int32
   return 0;
 }
 
+// Mode a convergence run takes that was tuned to per-phase launches.
+int rules_tuned_mode(const pgx_wiring* w, int32_t batch, int32_t n_it, int32_t t0,
+                     int32_t converge) {
+  Plan P;
+  int32_t kinds;
+  if (plan_of(w, &P, &kinds)) return -1;
+  Tuned tuned;
+  tuned.best.mode = 2;
+  tuned.task_loop.mode = 1;
+  return int(tuned_shape(tuned, converge != 0, P, kinds, batch, n_it, t0 != 0).mode);
+}
+
 // Patches of a graph: [patches, depth], or of one that only states its size
 // (w null): num_edges / 2 factors, and a task with none of them.
 int rules_patches(const pgx_wiring* w, int64_t num_edges, int64_t* out) {

@@ -222,6 +222,31 @@ def test_autotune_keeps_results(gpu):
 
 
 @pytest.mark.gpu
+def test_tuned_convergence_runs_do_not_launch_idle_iterations(gpu):
+  """A 100x100 torus may take per-phase launches for 300 iterations and not for
+  5,000, tuned with 10 or not: same results, and one launch of the task loop
+  for a run that stops at once."""
+  bb = batch.BatchedBP([batch.grid_wiring(100, 100, 2, torus=True, full_tables=True)],
+                       temperature=1.0)
+  rng = np.random.default_rng(4)
+  lp = rng.normal(0, 0.3, size=bb.layout.num_lp).astype(np.float32)
+  ev = rng.normal(size=bb.layout.num_vs).astype(np.float32)
+  before = [bb.run_converge(lp, None, ev, n, tol=1.0) for n in (300, 5000)]
+  bb.autotune(lp, None, ev, converge=True, probe_iters=10)
+  _lib.profile_kernels()
+  _lib.set_option("profile", 2)
+  for n, ref in zip((300, 5000), before):
+    res = bb.run_converge(lp, None, ev, n, tol=1.0)
+    kernels = _lib.profile_kernels()
+    assert all(np.array_equal(a.cpu().numpy(), b.cpu().numpy()) for a, b in zip(res, ref))
+    assert int(res[2][0]) < 10
+    if n == 5000:
+      assert set(kernels) == {"task_loop"} and kernels["task_loop"][1] == 1, kernels
+  _lib.profile_read()
+  bb.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("converge", [False, True])
 def test_autotune_of_a_graph_without_factors(gpu, converge):
   """Variables and no factors: every shape's run is empty, and one is chosen."""

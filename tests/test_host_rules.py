@@ -47,6 +47,18 @@ def test_convergence_shape_by_iterations_allowed(rules, side, n_it, want):
   assert _converge_shape(rules, torus, n_it)[1:] == want
 
 
+@pytest.mark.parametrize("n_it", [1, 10, 300, 480, 485, 5000])
+@pytest.mark.parametrize("side", [30, 100])
+def test_tuned_convergence_runs_follow_the_iterations_allowed(rules, side, n_it):
+  """Per-phase launches chosen by short probes run only where untuned runs of
+  as many iterations may take them; runs of a fixed count take them always."""
+  torus = batch.grid_wiring(side, side, 2, torus=True, full_tables=True)
+  w = torus.to_engine_wiring()
+  mode = lambda converge: rules.rules_tuned_mode(ctypes.byref(w.struct), 1, n_it, 0, converge)
+  assert mode(1) == _converge_shape(rules, torus, n_it)[1]
+  assert mode(0) == 2
+
+
 def test_patches_take_edge_numbers_of_28_bits(rules):
   """A patch's threads hold their edge in 28 bits under its ring: graphs with
   more edges have no patches, whatever their components' size."""
