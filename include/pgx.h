@@ -332,14 +332,18 @@ int64_t pgx_set_option(const char* key, int64_t value);
 
 /* With "profile" 1 or 2: waits for the recorded runs and returns the summed
  * GPU time of their BP iterations (milliseconds, HIP events on the run's
- * stream) and how many runs were recorded, then clears the record. */
+ * stream) and how many runs were recorded, then clears the record. The time
+ * holds the final messages' way into the caller's layout; the initial
+ * messages' normalisation (and packing to one float) comes before it, except
+ * in patches, whose launches read the caller's messages themselves. */
 int pgx_profile_read(double* total_ms, int64_t* num_runs);
 
 /* Kernel ids of pgx_profile_kernels. */
 #define PGX_KERNEL_TASK_LOOP 0
 #define PGX_KERNEL_VAR_PHASE 1
 #define PGX_KERNEL_VAR_COMBINE 2
-#define PGX_KERNEL_FAC_FUSED 3
+#define PGX_KERNEL_FAC_FUSED 3   /* also the launches of patches ("mode" 4), of up
+                                    to 4 iterations or a whole run each */
 #define PGX_KERNEL_FAC_PHASE 4   /* + block kind: 2x2 Enum, pairwise Enum,
                                     general Enum, OR, AND, Pool */
 #define PGX_KERNEL_BIPARTITE 10 /* complete bipartite binary graphs: whole iteration */
@@ -354,8 +358,8 @@ int pgx_profile_read(double* total_ms, int64_t* num_runs);
 /* With "profile" 2 every launch of pgx_run / pgx_run_converge (and of the
  * pairwise reverse pass of pgx_run_vjp) is bracketed
  * by HIP events on the run's stream (the back-to-back iteration launches of
- * the complete bipartite shape by one pair around all of them, so their
- * average includes the gaps between them but no event records). Fills total_ms[PGX_KERNEL_COUNT] and
+ * the complete bipartite shape and of patches by one pair around all of them,
+ * so their average includes the gaps between them but no event records). Fills total_ms[PGX_KERNEL_COUNT] and
  * launches[PGX_KERNEL_COUNT] (either may be NULL) with the summed GPU time
  * and launch count per kernel id since the last call, then clears them. */
 int pgx_profile_kernels(double* total_ms, int64_t* launches);

@@ -1007,7 +1007,7 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
       rc = t0 ? launch_coop<true>(g, r, batch, s, tile) : launch_coop<false>(g, r, batch, s, tile);
     });
   else if (mode == 4)
-    clk.run(PGX_KERNEL_FAC_FUSED, [&] {
+    clk.run_n(PGX_KERNEL_FAC_FUSED, patch_launches(g->patches.depth, n_it), [&] {
       rc = launch_patches(g, r, ftov_in, ftov_in_stride, ftov_out, scr, batch, t0, s);
     });
   else {

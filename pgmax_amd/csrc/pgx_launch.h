@@ -346,6 +346,9 @@ void launch_converge_finish(pgx_graph* g, const RunBufs& r, float* out, int32_t 
                             hipStream_t s);
 template <bool kT0>
 int launch_coop(pgx_graph* g, const RunBufs& r, int32_t batch, hipStream_t s, int64_t tile);
+inline int32_t patch_launches(int32_t depth, int32_t n_it) {
+  return depth ? (n_it + depth - 1) / depth : 1;
+}
 // pgx_patch.hip: a run in launches of patches.depth iterations (0: one launch),
 // from the caller's messages to the caller's result; buf holds two floats per
 // edge and batch element

@@ -244,6 +244,23 @@ def test_patches_match_oracle(gpu, kind, temperature, iters):
       np.testing.assert_array_equal(_np(od)[b], ref_d)
 
 
+@pytest.mark.parametrize("kind,iters,launches", [("whole", 9, 1), ("rings", 4, 1),
+                                                 ("rings", 5, 2), ("rings", 9, 3)])
+def test_patch_launches_are_counted(gpu, kind, iters, launches):
+  """The per-kernel record holds every launch of a run on patches."""
+  from pgmax_amd import engine
+  eng = engine.Engine.from_wiring(_binary_graph(kind).to_engine_wiring())
+  g = eng.graph
+  zeros = [np.zeros(n, np.float32) for n in (g.num_lp, g.num_es, g.num_vs)]
+  _lib.profile_kernels()
+  _lib.set_option("mode", 4)
+  _lib.set_option("profile", 2)
+  eng.run(*zeros, iters, 0.5, 1.0)
+  kernels = _lib.profile_kernels()
+  _lib.profile_read()
+  assert {k: n for k, (_, n) in kernels.items()} == {"fac_fused": launches}
+
+
 @pytest.mark.parametrize("kind", ["parents 1", "parents 2", "parents 3", "mixed", "wave"])
 @pytest.mark.parametrize("logical", ["or", "and"])
 @pytest.mark.parametrize("temperature", [0.0, 0.7])
