@@ -147,20 +147,23 @@ int pgx_run_converge(pgx_graph* graph,
                      int32_t batch, int32_t max_iters, float damping,
                      float temperature, float tol, void* stream);
 
-/* Autotuner: times every execution shape this graph allows (one workgroup
- * per task with 256 / 512 / 1024 threads, per-phase launches, with and
- * without factor-side variable sums and vector accesses) on the given
- * inputs for probe_iters iterations, and makes the fastest the graph's
- * shape for later pgx_run (converge = 0) or pgx_run_converge (converge = 1)
- * calls with the same batch size and temperature class (0 or > 0), as long
- * as the "mode", "block" and "tile" options are 0. Of a convergence run it
- * also keeps the fastest task-loop shape, which runs take whose max_iters
- * would leave too many per-phase launches idle after the last task stops. Per-phase shapes are
- * tried with 64, 128 and 256 factors per workgroup, the complete bipartite
- * iteration with tiles of 32 rows x 32, 64 or 128 columns and 256 or 512
- * threads, and per-phase runs with square pairwise tables both on S lanes
- * per factor and one factor per thread, with and without runs of
- * consecutive workgroups per XCD. chosen (7 int64, may be NULL) receives
+/* Autotuner: times execution shapes of this graph on the given inputs for
+ * probe_iters iterations and makes the fastest the graph's shape for later
+ * pgx_run (converge = 0) or pgx_run_converge (converge = 1) calls with the
+ * same batch size and temperature class (0 or > 0), as long as the "mode",
+ * "block" and "tile" options are 0. Timed are the shape an untuned run takes;
+ * one workgroup per task with 256 / 512 / 1024 threads, with and without
+ * factor-side variable sums; and, for fixed counts, per-phase launches with
+ * 64, 128 and 256 factors per workgroup, with and without factor-side
+ * variable sums and vector accesses, lane-group tiles of one and two passes
+ * where the graph is small, square pairwise tables on S lanes per factor and
+ * one factor per thread, runs of consecutive workgroups per XCD; one
+ * cooperative launch; patches; the complete bipartite iteration with tiles of
+ * 32 rows x 32, 64 or 128 columns and 256 or 512 threads. Convergence runs
+ * try per-phase launches where untuned ones of few enough iterations take
+ * them, and keep the fastest task-loop shape too, for runs whose max_iters
+ * would leave too many of those launches idle after the last task stops.
+ * chosen (7 int64, may be NULL) receives
  * [mode, block, fuse, vec, tile, lanes, xcd]. Synchronises the host. No
  * reference counterpart. */
 int pgx_autotune(pgx_graph* graph,

@@ -780,7 +780,10 @@ static size_t run_scratch_bytes(const pgx_graph* g, int32_t batch, int32_t n_it)
 }
 
 // Shared body of pgx_run and pgx_run_converge. With task_deltas set, the
-// run uses the task-loop shape and stops every task at its convergence.
+// run stops every task at its convergence, in the task loop or in per-phase
+// launches.
+// force: run in this shape (mode 0: the one the untuned rules choose);
+// taken: receives the shape the run took.
 // fixed_scratch (non-null): the run's scratch lies there (the caller checked
 // that run_scratch_bytes fits) instead of the graph's own, and the run makes
 // no allocation of any kind (no profiling events either).
@@ -789,7 +792,7 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
                     float* ftov_out, float* deltas, float* task_deltas, int32_t* iters_done,
                     int32_t batch, int32_t num_iters, float damping, float temperature, float tol,
                     void* stream, const RunCfg* force = nullptr,
-                    float* fixed_scratch = nullptr) {
+                    float* fixed_scratch = nullptr, RunCfg* taken = nullptr) {
   const bool converge = task_deltas != nullptr;
   if (!g || !ftov_out || batch <= 0 || (!converge && !deltas) || (converge && !iters_done))
     return set_error(PGX_EINVAL, "pgx_run: null argument or batch <= 0");
@@ -881,29 +884,24 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
     tile = g_opt_tile;
   }
   if (fixed_scratch) prof = 0;  // profiling events would be allocations
-  bool chosen = force != nullptr;  // shape set by the autotuner
-  if (force) {
-    mode = force->mode;
-    bs = force->bs;
-    fuse = force->fuse;
-    vec = force->vec;
-    tile = force->tile;
-    lanes = force->lanes;
-    xcd = force->xcd;
-  } else if (mode == 0 && bs == 0 && tile == 0) {
+  const RunCfg* cfg = force;  // shape set by the autotuner
+  if (!force && mode == 0 && bs == 0 && tile == 0) {
     auto it = g->tuned.find(std::make_tuple(batch, temperature == 0.f ? 1 : 0, converge ? 1 : 0));
-    if (it != g->tuned.end()) {
-      const RunCfg& c = tuned_shape(it->second, converge, g->plan, g->kinds_mask, batch, n_it,
-                                    temperature == 0.f);
-      mode = c.mode;
-      bs = c.bs;
-      fuse = c.fuse;
-      vec = c.vec;
-      tile = c.tile;
-      lanes = c.lanes;
-      xcd = c.xcd;
-      chosen = true;
-    }
+    if (it != g->tuned.end())
+      cfg = &tuned_shape(it->second, converge, g->plan, g->kinds_mask, batch, n_it,
+                         temperature == 0.f);
+  }
+  const bool chosen = cfg && cfg->mode != 0;
+  if (cfg) {
+    mode = cfg->mode;
+    bs = cfg->bs;
+    tile = cfg->tile;
+  }
+  if (chosen) {
+    fuse = cfg->fuse;
+    vec = cfg->vec;
+    lanes = cfg->lanes;
+    xcd = cfg->xcd;
   }
   const bool small_run =
       int64_t(batch) * d.num_es <= (g->kinds_mask == kKindsBin2 ? kFusedMaxBin2 : kFusedMaxStates);
@@ -977,6 +975,15 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
   // buffer, and the buffers swap roles, so iteration 0 reads the packed
   // messages and the last iteration writes r.x (unpacked into ftov_out below).
   g->dev.packed = (mode == 2 && !g->dev.bip && g->packed_plan && g->dev.even2 && pack) ? 1 : 0;
+  if (taken) {
+    const bool by_lanes = mode == 2 && g->dev.fusable && lanes && !g->dev.packed &&
+                          g->lsets[0].num_tiles > 0;
+    const bool threads = mode == 1 || (mode == 2 && g->dev.bip);
+    *taken = RunCfg{mode,  threads ? bs : 0,
+                    g->dev.fusable || g->dev.wide_fused || g->dev.bip ? 1 : 0,
+                    vec,   by_lanes ? 64 * kLaneFusedPasses[lset] / 4 : tile,
+                    lanes, mode == 2 ? r.xcd : 0};
+  }
   if (g->dev.packed) {
     std::swap(r.x, r.y);
     launch_pair_entry(g->dev, ftov_in, ftov_in_stride, nullptr, (n_it & 1) ? r.y : r.x, d.num_es,
@@ -1234,47 +1241,21 @@ int pgx_autotune(pgx_graph* g, const float* lp, int64_t lp_stride, const float* 
   const DevGraph& d = g->dev;
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int32_t n_it = std::max(probe_iters, 2);
-  std::vector<RunCfg> cands;
-  const bool can_fuse = g->fusable_plan || g->bip_plan || g->wide_plan;
-  const int64_t fuse_opts[2] = {can_fuse ? 1 : 0, 0};
-  const int nf = can_fuse ? 2 : 1;
-  for (int fi = 0; fi < nf; ++fi)
-    for (int64_t b : {256, 512, 1024}) cands.push_back(RunCfg{1, b, fuse_opts[fi], 3, 256});
-  if (!converge && g->bip_plan)  // k_bipartite tiles: (columns, threads)
-    for (const auto& ct : {std::make_pair(64, 256), std::make_pair(64, 512),
-                           std::make_pair(32, 256), std::make_pair(128, 512)})
-      cands.push_back(RunCfg{2, ct.second, 1, 3, ct.first});
-  if (!converge)
-    for (int fi = 0; fi < nf; ++fi) {
-      if (g->bip_plan && fuse_opts[fi]) continue;  // covered above
-      for (int64_t t : {64, 128, 256}) cands.push_back(RunCfg{2, 0, fuse_opts[fi], 3, t});
-      cands.push_back(RunCfg{2, 0, fuse_opts[fi], 0, 256});
-      // square pairwise tables: also thread per factor instead of S lanes
-      if (!fuse_opts[fi] && g->msets[2].kind_tile0[kPairLanesGroup + 1] >
-                                g->msets[2].kind_tile0[kPairLanesGroup])
-        for (int64_t t : {128, 256}) cands.push_back(RunCfg{2, 0, 0, 3, t, 0});
-      // runs of consecutive tiles per XCD (enough tiles for several rounds)
-      if (!fuse_opts[fi] && g->tsets[0].num_tiles >= 64 * 8)
-        for (int64_t x : {4, 16})
-          for (int64_t ln : {1, 0}) cands.push_back(RunCfg{2, 0, 0, 3, 256, ln, x});
-      // fused lane groups: also one factor per thread, and XCD runs
-      if (fuse_opts[fi] && g->lsets[0].num_tiles > 0) {
-        if (lane_sets_from(g, batch) == 0)
-          for (int64_t t : {16, 32}) cands.push_back(RunCfg{2, 0, 1, 3, t});
-        cands.push_back(RunCfg{2, 0, 1, 3, 256, 0, 0});
-        for (int64_t x : {4, 16}) cands.push_back(RunCfg{2, 0, 1, 3, 256, 1, x});
-      }
-    }
-  // per-phase launches that skip the tasks that are done, where untuned runs
-  // of few enough iterations take them (tuned_shape looks at each run's count)
-  if (converge && converge_shape(g->plan, g->kinds_mask, batch, 1, temperature == 0.f).first == 2)
-    for (int fi = g->fusable_plan ? 0 : 1; fi < 2; ++fi)
-      for (int64_t t : {64, 128, 256}) cands.push_back(RunCfg{2, 0, fi == 0 ? 1 : 0, 3, t});
-  if (!converge && g->patches.count > 0) cands.push_back(RunCfg{4, 0, 1, 3, 256});
-  if (!converge && g->fusable_plan)
-    for (int64_t t : {64, 256}) cands.push_back(RunCfg{3, 0, 1, 3, t});
-  // the task loop last, so its probes can stop early against the best shape
-  std::stable_partition(cands.begin(), cands.end(), [](const RunCfg& c) { return c.mode != 1; });
+  TuneInput in;
+  in.converge = converge != 0;
+  in.bipartite = g->bip_plan != 0;
+  in.fusable = g->fusable_plan != 0;
+  in.wide = g->wide_plan != 0;
+  in.logical = (g->kinds_mask & ((1 << kOr) | (1 << kAnd))) != 0;
+  in.patches = g->patches.count > 0;
+  in.square = g->msets[2].kind_tile0[kPairLanesGroup + 1] > g->msets[2].kind_tile0[kPairLanesGroup];
+  in.lane_tiles = g->lsets[0].num_tiles > 0;
+  in.short_lane_tiles = in.lane_tiles && lane_sets_from(g, batch) == 0;
+  in.tiles = g->tsets[0].num_tiles;
+  in.per_phase_converge =
+      in.converge &&
+      converge_shape(g->plan, g->kinds_mask, batch, 1, temperature == 0.f).first == 2;
+  const std::vector<RunCfg> cands = tune_candidates(in);
   float *out = nullptr, *dl = nullptr;
   int32_t* it_done = nullptr;
   const size_t out_bytes = size_t(batch) * size_t(std::max<int64_t>(d.num_es, 1)) * 4;
@@ -1292,6 +1273,7 @@ int pgx_autotune(pgx_graph* g, const float* lp, int64_t lp_stride, const float* 
   if (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)
     rc = set_error(PGX_EHIP, "pgx_autotune: hipEventCreate failed");
   Tuned tuned;
+  RunCfg untuned{1, 256};  // what the untuned rules take (a run of no factors takes nothing)
   float best_ms = 3.4e38f, loop_ms = 3.4e38f;
   for (const RunCfg& c : cands) {
     if (rc) break;
@@ -1300,10 +1282,10 @@ int pgx_autotune(pgx_graph* g, const float* lp, int64_t lp_stride, const float* 
       (void)hipEventRecord(e0, s);
       rc = converge ? run_impl(g, lp, lp_stride, ev, ev_stride, ftov_in, ftov_in_stride, out,
                                nullptr, dl, it_done, batch, n_it, damping, temperature, 0.f,
-                               stream, &c)
+                               stream, &c, nullptr, c.mode == 0 ? &untuned : nullptr)
                     : run_impl(g, lp, lp_stride, ev, ev_stride, ftov_in, ftov_in_stride, out, dl,
                                nullptr, nullptr, batch, n_it, damping, temperature, 0.f, stream,
-                               &c);
+                               &c, nullptr, c.mode == 0 ? &untuned : nullptr);
       (void)hipEventRecord(e1, s);
       if (rc) break;
       if (hipEventSynchronize(e1) != hipSuccess) {
@@ -1336,7 +1318,7 @@ int pgx_autotune(pgx_graph* g, const float* lp, int64_t lp_stride, const float* 
   if (rc) return rc;
   g->tuned[std::make_tuple(batch, temperature == 0.f ? 1 : 0, converge ? 1 : 0)] = tuned;
   if (chosen) {
-    const RunCfg& best = tuned.best;
+    const RunCfg& best = tuned.best.mode == 0 ? untuned : tuned.best;
     chosen[0] = best.mode;
     chosen[1] = best.bs;
     chosen[2] = best.fuse;

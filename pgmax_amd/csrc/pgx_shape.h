@@ -4,13 +4,16 @@
 #define PGX_SHAPE_H_
 
 #include <utility>
+#include <vector>
 
 #include "pgx_plan.h"
 
 namespace pgx {
 
-// Execution shape of one run: mode 1 task loop / 2 phased, workgroup size of
-// the task loop, factor-side variable sums, vector accesses.
+// Execution shape of one run: mode 1 task loop / 2 phased / 3 cooperative / 4
+// patches, workgroup size of the task loop and of the bipartite tiles,
+// factor-side variable sums, vector accesses. mode 0: the untuned rules choose,
+// under the options in force.
 struct RunCfg {
   int64_t mode = 0, bs = 0, fuse = 1, vec = 3, tile = 256, lanes = 1, xcd = 0;
 };
@@ -46,6 +49,26 @@ struct Tuned {
 // task loop elsewhere.
 const RunCfg& tuned_shape(const Tuned& tuned, bool converge, const Plan& plan, int32_t kinds_mask,
                           int32_t batch, int32_t n_it, bool t0);
+
+// What the autotuner's shapes depend on.
+struct TuneInput {
+  bool converge = false;
+  bool bipartite = false;           // complete bipartite binary graph
+  bool fusable = false;             // factor side may form the variable sums
+  bool wide = false;                // pairwise tables above 8 states that may
+  bool logical = false;             // OR or AND factors
+  bool patches = false;
+  bool square = false;              // square pairwise tables of 3..8 states
+  bool lane_tiles = false;          // fused lane-group tiles
+  bool short_lane_tiles = false;    // those of one and two passes, at this batch size
+  bool per_phase_converge = false;  // converge_shape takes per-phase launches for some n_it
+  int32_t tiles = 0;                // per-phase tiles of 64 factors
+};
+// The shapes the autotuner times, the task loop's last so that their probes can
+// stop early against the best of the others. The untuned rules' own choice is
+// always among them (RunCfg{} with tile 0): they also take shapes no list names
+// for every graph, and a tuned graph must not run slower than an untuned one.
+std::vector<RunCfg> tune_candidates(const TuneInput& in);
 
 }  // namespace pgx
 

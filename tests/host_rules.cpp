@@ -46,6 +46,24 @@ int rules_tuned_mode(const pgx_wiring* w, int32_t batch, int32_t n_it, int32_t t
   return int(tuned_shape(tuned, converge != 0, P, kinds, batch, n_it, t0 != 0).mode);
 }
 
+// The autotuner's shapes, 7 numbers each (as pgx_autotune returns them), at
+// most `most` of them; flags: TuneInput's in order, bit by bit. Returns their
+// number.
+int rules_candidates(int32_t flags, int32_t tiles, int64_t* out, int32_t most) {
+  TuneInput in;
+  bool* const f[] = {&in.converge, &in.bipartite, &in.fusable,    &in.wide,
+                     &in.logical,  &in.patches,   &in.square,     &in.lane_tiles,
+                     &in.short_lane_tiles,        &in.per_phase_converge};
+  for (int k = 0; k < 10; ++k) *f[k] = (flags >> k) & 1;
+  in.tiles = tiles;
+  const std::vector<RunCfg> c = tune_candidates(in);
+  for (int i = 0; i < int(c.size()) && i < most; ++i) {
+    const int64_t v[] = {c[i].mode, c[i].bs, c[i].fuse, c[i].vec, c[i].tile, c[i].lanes, c[i].xcd};
+    for (int k = 0; k < 7; ++k) out[7 * i + k] = v[k];
+  }
+  return int(c.size());
+}
+
 // Patches of a graph: [patches, depth], or of one that only states its size
 // (w null): num_edges / 2 factors, and a task with none of them.
 int rules_patches(const pgx_wiring* w, int64_t num_edges, int64_t* out) {

@@ -59,6 +59,37 @@ def test_tuned_convergence_runs_follow_the_iterations_allowed(rules, side, n_it)
   assert mode(0) == 2
 
 
+_FLAGS = ("converge", "bipartite", "fusable", "wide", "logical", "patches", "square",
+          "lane_tiles", "short_lane_tiles", "per_phase_converge")
+
+
+def _candidates(rules, *names, tiles=100):
+  out = (ctypes.c_int64 * (7 * 64))()
+  n = rules.rules_candidates(sum(1 << _FLAGS.index(k) for k in names), tiles, out, 64)
+  assert n <= 64
+  return [tuple(out[7 * i:7 * i + 7]) for i in range(n)]
+
+
+def test_autotuner_times_what_untuned_runs_take(rules):
+  """(mode, threads, fuse, vec, tile, lanes, xcd): mode 0 is the untuned rules'
+  own choice, in every list; the shapes those rules take by name are listed too,
+  and task loops come last."""
+  for flags in range(1 << len(_FLAGS)):
+    names = [k for i, k in enumerate(_FLAGS) if flags >> i & 1]
+    got = _candidates(rules, *names, tiles=(0, 600)[flags & 1])
+    assert got.count((0, 0, 1, 3, 0, 1, 0)) == 1
+    assert len(set(got)) == len(got)
+    modes = [c[0] for c in got]
+    assert modes.count(1) == modes[::-1].index(next(m for m in modes[::-1] if m != 1)) >= 3
+    if "converge" in names:
+      assert set(modes) <= {0, 1, 2} and (2 in modes) == ("per_phase_converge" in names)
+  assert (2, 512, 1, 3, 32, 1, 0) in _candidates(rules, "bipartite")
+  assert (2, 0, 0, 3, 256, 1, 8) in _candidates(rules, "logical", tiles=8)
+  for t in (16, 32):
+    assert (2, 0, 1, 3, t, 1, 0) in _candidates(rules, "converge", "fusable", "lane_tiles",
+                                                "short_lane_tiles", "per_phase_converge")
+
+
 def test_patches_take_edge_numbers_of_28_bits(rules):
   """A patch's threads hold their edge in 28 bits under its ring: graphs with
   more edges have no patches, whatever their components' size."""
