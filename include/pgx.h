@@ -287,7 +287,8 @@ int pgx_enum_rows_fac_to_var(const int32_t* cfg_row_ptr, const int32_t* row_es,
  * factor side recomputes variable sums, see "fuse", 4 patches: small graphs of
  * 2x2 factors, several iterations per launch), "block" (threads per
  * workgroup of the task loop and of the complete bipartite iteration:
- * 128, 256 or 512 there, 0 auto), "profile" (1: record
+ * 128, 256 or 512 there; 0 auto: 512 there for at most 512 tiles of 32
+ * columns), "profile" (1: record
  * HIP events around the BP iterations of every pgx_run; 2: also around every
  * kernel launch), "fuse" (1, the
  * default: graphs of pairwise factors whose variables have at most 8 edges

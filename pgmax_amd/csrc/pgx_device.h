@@ -1527,6 +1527,15 @@ __device__ void logical_factor_wide(const DevGraph& g, int32_t f, int32_t off, c
                   q == 0, dl);
 }
 
+// A value from the lane before, within a row of 16 lanes.
+__device__ __forceinline__ float lane_before(float x) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x111, 0xf, 0xf, false));
+}
+__device__ __forceinline__ float read_lane(float x, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
+}
+
 // A logical factor of at most kWaveParents parents on one wavefront: lane L
 // takes parents 4L .. 4L + 3, so a run of kVarChunk parents is eight
 // consecutive lanes and every load of the wavefront is one contiguous
@@ -1547,14 +1556,6 @@ static_assert(kWaveParents == kWaveLogicalParents && kVarChunk % kWaveItems == 0
 // message is kept for the damping (four floats one by one, and the message
 // again for the output: 9,600 OR factors of up to 180 parents 31 us an
 // iteration, now 27.7).
-// A value from the lane before, within a row of 16 lanes.
-__device__ __forceinline__ float lane_before(float x) {
-  return __int_as_float(
-      __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x111, 0xf, 0xf, false));
-}
-__device__ __forceinline__ float read_lane(float x, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), lane));
-}
 template <class IO>
 __device__ __forceinline__ void logical_factor_wave(const DevGraph& g, int32_t f, int32_t off,
                                                     const IO& io, float t, bool normalize,

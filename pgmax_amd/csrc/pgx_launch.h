@@ -93,9 +93,12 @@ constexpr int32_t kPairWideTile = -64;  // Tile::pad of tiles run by pair_wide (
 constexpr int32_t kBin2PerThread = 4;  // 2x2 factors per thread in k_fac_phase (msets tiles)
 // Untuned, one launch per iteration (variable sums on the factor side) up to
 // this many edge states per run. 2x2 factors: every thread re-reads the 8
-// messages around its factor, which from about 2^21 edge states on costs more
-// than the second launch (128 x 128 tori, us an iteration: 4 of them 7.5
-// against 10.8, 16 15.3 against 13.8, 96 57.5 against 43.3). Square tables
+// messages around its factor, which from about 1.5 * 2^20 edge states on costs
+// more than the second launch (us an iteration against two launches, T = 1:
+// 128 x 128 tori of 2^17 edge states each, 8 of them 8.9 and 9.7, 10 9.9 and
+// 9.9, 12 10.5 and 10.2, 14 11.0 and 10.6, 16 13.8 and 12.0, 96 57.5 and 43.3;
+// 48 x 48 tori, 1.25 * 2^20 8.9 and 9.7, 1.5 9.6 and 9.8, 1.74 10.2 and 10.5,
+// 2 12.6 and 12.4; T = 0 crosses between 1.75 and 2 * 2^20). Square tables
 // share these sums among more work (64 Potts grids up to 110 x 110 x 8, 7
 // million edge states, 49 against 62; 256 grids, 32 million, 221 against 218).
 constexpr int64_t kFusedMaxBin2 = int64_t(3) << 19;

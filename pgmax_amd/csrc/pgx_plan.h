@@ -1,6 +1,6 @@
 // Host-side compilation of the reference's flat wiring into the engine's
 // device layout ("plan"). Shared between the plan compiler (pgx_plan.cpp)
-// and the kernels (pgx_kernels.hip).
+// and the kernels (pgx_device.h).
 #ifndef PGX_PLAN_H_
 #define PGX_PLAN_H_
 
@@ -125,7 +125,7 @@ struct Plan {
   // row_desc in the order of heavy_col_chunks / heavy_row_chunks.
   std::vector<int32_t> chunk_desc, chunk_desc_ref, col_desc, row_desc;
   // Heavy-variable descriptors, 4 ints each: [first variable state,
-  // chunks | ns << 16, first chunk slot, 0].
+  // chunks | ns << 16, first chunk slot, padding to one 16-byte load].
   std::vector<int32_t> heavy_desc;
   // Variables of more than kThreadStates states and at most kVarChunk edges,
   // 4 ints each: [first variable state, states, first adjacency index, edges].
