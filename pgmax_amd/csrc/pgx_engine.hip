@@ -976,12 +976,13 @@ static int run_impl(pgx_graph* g, const float* lp, int64_t lp_stride, const floa
   // messages and the last iteration writes r.x (unpacked into ftov_out below).
   g->dev.packed = (mode == 2 && !g->dev.bip && g->packed_plan && g->dev.even2 && pack) ? 1 : 0;
   if (taken) {
-    const bool by_lanes = mode == 2 && g->dev.fusable && lanes && !g->dev.packed &&
-                          g->lsets[0].num_tiles > 0;
-    const bool threads = mode == 1 || (mode == 2 && g->dev.bip);
-    *taken = RunCfg{mode,  threads ? bs : 0,
-                    g->dev.fusable || g->dev.wide_fused || g->dev.bip ? 1 : 0,
-                    vec,   by_lanes ? 64 * kLaneFusedPasses[lset] / 4 : tile,
+    const bool bip = mode == 2 && g->dev.bip;
+    int64_t t = tile;
+    if (bip && tile > 128) t = 32;  // (columns; launch_bipartite's default)
+    if (mode == 2 && g->dev.fusable && lanes && !g->dev.packed && g->lsets[0].num_tiles > 0)
+      t = 16 * kLaneFusedPasses[lset];
+    *taken = RunCfg{mode,  mode == 1 || bip ? bs : 0,
+                    bip || g->dev.fusable || g->dev.wide_fused ? 1 : 0, vec, t,
                     lanes, mode == 2 ? r.xcd : 0};
   }
   if (g->dev.packed) {
