@@ -1126,6 +1126,19 @@ __device__ __forceinline__ void pair_wide(const DevGraph& g, const Block& b, int
 // summaries (s0 s1 <= 1,024, an odd pitch adds at most one float per row).
 constexpr int kPairWideLds = 64 + 1024 + 64;
 
+// The compiled topology, which no kernel writes, in the constant address space:
+// an element whose index is the same in every lane is one scalar load. From
+// global memory the compiler makes that of it only while it can prove that no
+// store of the kernel comes before, which it gives up in larger kernels: when
+// pair_wide joined the general kernel, a 24 x 24 grid of 33 states went from 5.4
+// to 8.7 ms an iteration at T = 0, 1,500 triples of 6 configs from 38 to 48 us
+// (T = 1, whose loads it never proved: 17.5 ms and 78 us). Now 5.4 ms and 38 us
+// (T = 1: 10.8 and 59).
+typedef const __attribute__((address_space(4))) int32_t* ConstInts;
+__device__ __forceinline__ ConstInts const_ints(const int32_t* p) {
+  return (ConstInts)reinterpret_cast<uintptr_t>(p);
+}
+
 // Any Enum factor: config table in `tables` as [nv edge offsets][esf owning
 // edge][nc * nv edge-state offsets]; summaries are recomputed per edge state
 // instead of being stored, so no per-thread arrays are needed.
@@ -1136,9 +1149,9 @@ __device__ void enum_general(const DevGraph& g, const Block& b, int32_t i, const
   const int32_t es0 = b.es0 + esf * i;
   const int32_t e0 = b.e0 + nv * i;
   const int32_t c0 = b.c0 + nc * i;
-  const int32_t* eoff = g.tables + b.tbl;
-  const int32_t* owner = eoff + nv;
-  const int32_t* rows = owner + esf;
+  const ConstInts eoff = const_ints(g.tables) + b.tbl;
+  const ConstInts owner = eoff + nv;
+  const ConstInts rows = owner + esf;
   auto row_vt = [&](int32_t k) {
     const int32_t j = owner[k];
     return io.vt(g.edge_vs0[e0 + j] + (k - eoff[j]), es0 + k);
